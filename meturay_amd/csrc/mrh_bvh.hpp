@@ -53,11 +53,18 @@ int32_t lbvh_create(mrh_context* ctx, const float* d_tris, uint32_t n, uint32_t 
 int32_t lbvh_build_into(mrh_lbvh* b, const float* d_tris);
 void lbvh_free(mrh_lbvh* b);
 
+// Rays a wave starts with when there are few: a launch whose rays leave
+// waves free gives each wave 32 or 16 of them instead of 64, so a wave waits
+// for the longest of fewer rays (walk4_stream).  16 measured best: guided
+// 1024x768 renders 19.29 / 18.99 / 18.81 / 18.88 ms at 64 / 32 / 16 / 8.
+constexpr uint32_t TRACE_MIN_GROUP = 16;
+
 // Persistent grid of the traversal kernels: a multiple of 8 blocks (one
-// slice per XCD) of `block` threads.
+// slice per XCD) of `block` threads, with room for waves of
+// TRACE_MIN_GROUP rays.
 inline uint32_t trace_grid(mrh_context* ctx, uint64_t rays, uint32_t block = 256)
 {
-    uint64_t want = (rays + block - 1) / block;
+    uint64_t want = (rays * (64 / TRACE_MIN_GROUP) + block - 1) / block;
     uint64_t cap = (uint64_t)ctx->num_cus * ctx->trace_blocks_per_cu;
     if (want > cap) want = cap;
     want = (want + 7) & ~7ull;
@@ -138,10 +145,10 @@ struct PrivateStack {
     }
 };
 
-// LDS pointers with their address space spelled out, so no access through
-// them is compiled as a generic (flat) access.
-typedef __attribute__((address_space(3))) uint32_t lds_u32;
-typedef __attribute__((address_space(3))) float lds_f32;
+// An LDS pointer with its address space spelled out, so no access through it
+// is compiled as a generic (flat) access.
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) u32x2 lds_u32x2;
 
 // Waves per SIMD a trace kernel asks the register allocator for: `want`,
 // or fewer when its LDS stack (L entries of 8 bytes per thread, BLOCK
@@ -159,37 +166,34 @@ template <int L, int N, int BLOCK>
 struct LdsStack {
     static constexpr int CAP = N;
     static constexpr int LDS_ENTRIES = L;
-    lds_u32* s_node;      // [L][BLOCK]
-    lds_f32* s_t;         // [L][BLOCK]
+    lds_u32x2* s;         // [L][BLOCK] (code, entry distance)
     uint32_t slot;        // threadIdx.x
-    uint2* overflow;      // [(N-L)][ostride]
-    size_t ostride, oslot;
-    __device__ __forceinline__ LdsStack(uint32_t* node, float* t, uint32_t sl, uint2* ovf, size_t ost, size_t osl)
-        : s_node((lds_u32*)node), s_t((lds_f32*)t), slot(sl), overflow(ovf), ostride(ost), oslot(osl)
+    uint2* overflow;      // this thread's slice, [N - L]
+    __device__ __forceinline__ LdsStack(u32x2* entries, uint32_t sl, uint2* ovf, size_t oslot)
+        : s((lds_u32x2*)entries), slot(sl), overflow(ovf + oslot * (size_t)(N > L ? N - L : 0))
     {
     }
     __device__ __forceinline__ void put(int i, uint32_t n, float d)
     {
         if (i < L) {
-            s_node[i * BLOCK + slot] = n;
-            s_t[i * BLOCK + slot] = d;
+            put_lds(i, n, d);
         } else {
-            overflow[(size_t)(i - L) * ostride + oslot] = make_uint2(n, __float_as_uint(d));
+            overflow[i - L] = make_uint2(n, __float_as_uint(d));
         }
     }
     // entry i < L, no check
     __device__ __forceinline__ void put_lds(int i, uint32_t n, float d)
     {
-        s_node[i * BLOCK + slot] = n;
-        s_t[i * BLOCK + slot] = d;
+        s[i * BLOCK + slot] = u32x2{n, __float_as_uint(d)};
     }
     __device__ __forceinline__ void get(int i, uint32_t& n, float& d) const
     {
         if (i < L) {
-            n = s_node[i * BLOCK + slot];
-            d = s_t[i * BLOCK + slot];
+            const u32x2 e = s[i * BLOCK + slot];
+            n = e.x;
+            d = __uint_as_float(e.y);
         } else {
-            const uint2 e = overflow[(size_t)(i - L) * ostride + oslot];
+            const uint2 e = overflow[i - L];
             n = e.x;
             d = __uint_as_float(e.y);
         }
@@ -496,6 +500,212 @@ __device__ __forceinline__ TraceResult traverse4(Stack& st, const float4* __rest
         }
         if (STATS) r.visits++;
         next = node4_order_push(st, sp, node4_test(nbase, next << 7, sl, tmin, r.t));
+    }
+}
+
+// node4_order_push in fewer operations: the same order (entry distance, then
+// slot), from a 5-comparator network that carries no slot numbers.  The first
+// four exchanges keep equal distances in slot order by themselves (they
+// compare neighbours, or the first against the second pair); in the last one
+// a tie puts the element from the first pair's back half before the second
+// pair's front only where neither of the cross exchanges swapped.  The
+// nearest slot's entry distance goes to dist.
+template <class Stack>
+__device__ __forceinline__ uint32_t node4_near_push(Stack& st, int& sp, const Node4Test& q, float& dist)
+{
+    float k0 = q.h0 ? q.k.x : INFINITY, k1 = q.h1 ? q.k.y : INFINITY, k2 = q.h2 ? q.k.z : INFINITY,
+          k3 = q.h3 ? q.k.w : INFINITY;
+    uint32_t c0 = q.c.x, c1 = q.c.y, c2 = q.c.z, c3 = q.c.w;
+    auto cx = [](bool sw, float& ka, uint32_t& ca, float& kb, uint32_t& cb) {
+        const float tk = sw ? kb : ka;
+        kb = sw ? ka : kb;
+        ka = tk;
+        const uint32_t tc = sw ? cb : ca;
+        cb = sw ? ca : cb;
+        ca = tc;
+    };
+    cx(k1 < k0, k0, c0, k1, c1);
+    cx(k3 < k2, k2, c2, k3, c3);
+    const bool sa = k2 < k0, sb = k3 < k1;
+    cx(sa, k0, c0, k2, c2);
+    cx(sb, k1, c1, k3, c3);
+    cx((k2 < k1) | ((sa | sb) & (k2 == k1)), k1, c1, k2, c2);
+    dist = k0;
+    if constexpr (Stack::LDS_ENTRIES >= 3) {
+        if (sp + 3 <= Stack::LDS_ENTRIES) {   // room for three entries in the LDS part
+            if (k3 < INFINITY) st.put_lds(sp++, c3, k3);
+            if (k2 < INFINITY) st.put_lds(sp++, c2, k2);
+            if (k1 < INFINITY) st.put_lds(sp++, c1, k1);
+            return k0 < INFINITY ? c0 : NO_HIT;
+        }
+    }
+    // the guard keeps a malformed tree from writing past the stack (the
+    // host sizes CAP for the tree depth)
+    if (k3 < INFINITY && sp < Stack::CAP) st.put(sp++, c3, k3);
+    if (k2 < INFINITY && sp < Stack::CAP) st.put(sp++, c2, k2);
+    if (k1 < INFINITY && sp < Stack::CAP) st.put(sp++, c1, k1);
+    return k0 < INFINITY ? c0 : NO_HIT;
+}
+
+// One lane's state in walk4_stream: traverse4's walk with leaves put off.
+// `next` is the node to test, or a leaf that waits behind `pend`, the leaf to
+// test next; both carry their entry distance.
+struct Walk4 {
+    V3 o, d;
+    RaySlab sl;
+    uint32_t next, pend;
+    float next_t, pend_t;
+    int sp;
+    float t;
+    uint32_t leaf;
+    float ba, bb;
+    __device__ __forceinline__ void begin(V3 ro, V3 rd, float tmax, uint32_t root)
+    {
+        o = ro;
+        d = rd;
+        sl = make_slab(o, d);
+        next = root;
+        pend = NO_HIT;
+        next_t = pend_t = -INFINITY;
+        sp = 0;
+        t = tmax;
+        leaf = NO_HIT;
+        ba = bb = 0.0f;
+    }
+    // a leaf in `next` moves to a free `pend` (NO_HIT and out-of-range codes
+    // are no leaf)
+    __device__ __forceinline__ void stash(uint32_t n_leaves)
+    {
+        const uint32_t li = next ^ LEAF_BIT;
+        const bool put = li < n_leaves && pend == NO_HIT;
+        pend = put ? li : pend;
+        pend_t = put ? next_t : pend_t;
+        next = put ? NO_HIT : next;
+    }
+    // at most one pop: a second one in the same step would keep the wave's
+    // other lanes waiting for the few that need it
+    template <class Stack>
+    __device__ __forceinline__ void settle(const Stack& st, uint32_t n_leaves)
+    {
+        stash(n_leaves);
+        if (next == NO_HIT && sp > 0) {
+            --sp;
+            uint32_t nn;
+            st.get(sp, nn, next_t);
+            next = (next_t > t) ? NO_HIT : nn;
+            stash(n_leaves);
+        }
+    }
+    template <bool ANY>
+    __device__ __forceinline__ void test_leaf(const float4* __restrict__ leaves, float tmin)
+    {
+        const uint32_t li = pend;
+        pend = NO_HIT;
+        const float4 a = leaves[3 * (size_t)li + 0];
+        const float4 b = leaves[3 * (size_t)li + 1];
+        const float4 c = leaves[3 * (size_t)li + 2];
+        float tt, na, nb;
+        const bool in = intersect_tri_flat(o, d, v3(a.x, a.y, a.z), v3(b.x, b.y, b.z), v3(c.x, c.y, c.z), tt, na, nb);
+        const bool hit = in & (tt >= tmin) & (tt < t) & !(pend_t > t);
+        leaf = hit ? li : leaf;
+        ba = hit ? na : ba;
+        bb = hit ? nb : bb;
+        t = hit ? tt : t;
+        if (ANY) {   // the walk of this ray is over
+            next = hit ? NO_HIT : next;
+            sp = hit ? 0 : sp;
+        }
+    }
+};
+
+__device__ __forceinline__ uint32_t rank_below(uint64_t mask)
+{
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+
+// Lanes without a ray at which a wave takes new rays.  1080p frame of the
+// 2 M-triangle sphere grid: 15.3 / 14.8 / 14.5 / 14.6 ms at 32 / 40 / 48 /
+// 56 (never, 64: 15.4); 4 M random rays through 1 M triangles, closest and
+// any: 7.11 / 7.02 / 7.06 / 7.20 ms (never: 9.2).  Refilling earlier keeps
+// more lanes busy but spreads a wave's node fetches over more cache lines.
+constexpr uint32_t WALK_REFILL = 48;
+
+// Closest / any hits of rays [0, n) over the 4-wide tree, for a wave of a
+// persistent grid of `waves`: rays group, group + stride, ... in groups of G
+// (64; 32 or 16 when there are fewer rays than lanes).  fetch(i, o, d, tmax)
+// reads ray i, emit(i, leaf, t, ba, bb) takes its result.
+//
+// Every ray is walked in traverse4's order, with two changes in how the
+// wave's lanes take their turns:
+//  * Leaves are put off: a lane that comes to a leaf keeps it in `pend` and
+//    walks on, up to its second leaf.  The wave tests nodes while at least
+//    5/8 of the lanes with work can, else the pending leaves.  traverse4 ran
+//    its leaf test for 8 of 64 lanes on average, this runs it for 16 to 25.
+//  * Lanes that are done take new rays once WALK_REFILL of them are.
+// A pending leaf is tested in its turn, and only if its entry distance is
+// still within the closest hit, which is what traverse4 decides when it pops
+// it; nodes may be visited that traverse4 had dropped by then, and any leaf
+// under such a node lies beyond the closest hit too.  So the hits are
+// traverse4's, bit for bit, ties included (its STATS walk counts visits).
+//
+// Each step ends: a node or leaf step works for at least one lane, or all
+// lanes with work hold stack entries only, of which every step pops one.
+//
+// Bound by the node fetches (seven 16-byte loads of 64 lanes each keep the
+// CU's address unit 70 % busy) and by VALU issue (75 %).  Against the
+// one-ray-per-lane loop over traverse4: the frame above 16.5 -> 14.5 ms, the
+// casts 11.0 -> 6.6 ms.
+template <bool ANY, class Stack, class Fetch, class Emit>
+__device__ __forceinline__ void walk4_stream(Stack& st, const float4* __restrict__ nodes4,
+                                             const float4* __restrict__ leaves, uint32_t root, uint32_t n_leaves,
+                                             float tmin, uint32_t wave, uint32_t waves, uint32_t n, Fetch&& fetch,
+                                             Emit&& emit)
+{
+    uint32_t G = 64u;
+    while (G > TRACE_MIN_GROUP && (uint64_t)waves * (G >> 1) >= n) G >>= 1;
+    const uint32_t stride = waves * G;
+    const char* nbase = (const char*)nodes4;
+    const uint32_t n_int = n_leaves - 1u;
+    uint32_t group = __builtin_amdgcn_readfirstlane(wave) * G, used = 0;   // next rays of the wave
+    uint32_t ray = NO_HIT;
+    Walk4 w;
+    w.begin(v3(0.0f, 0.0f, 0.0f), v3(0.0f, 0.0f, 0.0f), 0.0f, NO_HIT);
+    for (;;) {
+        uint64_t ma;
+        for (;;) {
+            w.settle(st, n_leaves);
+            const bool can = w.next < n_int;
+            const uint64_t mc = __ballot(can), mp = __ballot(w.pend != NO_HIT);
+            ma = mc | mp | __ballot(w.sp > 0);
+            if ((uint32_t)__popcll(ma) <= 64u - WALK_REFILL && (group < n || !ma)) break;
+            if (!mp || 8u * (uint32_t)__popcll(mc) >= 5u * (uint32_t)__popcll(ma)) {
+                if (can) w.next = node4_near_push(st, w.sp, node4_test(nbase, w.next << 7, w.sl, tmin, w.t), w.next_t);
+            } else {
+                if (w.pend != NO_HIT) w.test_leaf<ANY>(leaves, tmin);
+            }
+        }
+        const bool dead = !(w.next < n_int || w.pend != NO_HIT || w.sp > 0);
+        if (dead && ray != NO_HIT) {
+            emit(ray, w.leaf, w.t, w.ba, w.bb);
+            ray = NO_HIT;
+        }
+        if (group >= n) break;
+        if (dead) {
+            const uint32_t q = used + rank_below(~ma);
+            const uint32_t i = group + q + (q >= G ? stride - G : 0u);
+            if (i < n) {
+                V3 o, d;
+                float tmax;
+                fetch(i, o, d, tmax);
+                w.begin(o, d, tmax, root);
+                ray = i;
+            }
+        }
+        used += (uint32_t)__popcll(~ma);
+        if (used >= G) {
+            used -= G;
+            group += stride;
+        }
     }
 }
 

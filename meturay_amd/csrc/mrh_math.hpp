@@ -315,6 +315,27 @@ MRH_HD bool intersect_tri(V3 o, V3 d, V3 p0, V3 p1, V3 p2, float& t, float& ba, 
     return true;
 }
 
+// intersect_tri without early exits: the same operations and the same
+// outcome, all conditions tested at the end.  For a wave some lane nearly
+// always takes every step, so the exits only cost branches.
+MRH_HD bool intersect_tri_flat(V3 o, V3 d, V3 p0, V3 p1, V3 p2, float& t, float& ba, float& bb)
+{
+    const V3 e0 = p1 - p0;
+    const V3 e1 = p2 - p0;
+    const V3 p = cross(d, e1);
+    const float det = dot(e0, p);
+    const float inv_det = 1.0f / det;
+    const V3 tv = o - p0;
+    const float u = dot(tv, p) * inv_det;
+    const V3 q = cross(tv, e0);
+    const float v = dot(d, q) * inv_det;
+    const float tt = dot(e1, q) * inv_det;
+    t = tt;
+    ba = 1.0f - u - v;
+    bb = u;
+    return !(fabsf(det) < 1.0e-7f) & !(u < 0.0f) & !(u > 1.0f) & !(v < 0.0f) & !((v + u) > 1.0f) & !(tt <= 1.0e-7f);
+}
+
 // RayLib/Ray.hpp:248-270 slab test with IEEE minNum/maxNum.
 MRH_HD bool intersect_box(V3 o, V3 inv_d, float bx0, float by0, float bz0, float bx1,
                           float by1, float bz1, float tmin, float tmax, float& t_enter)

@@ -56,19 +56,35 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(lds_stack_wa
                                                   uint32_t bounce, float tmin, float tmax, HitBuf hit,
                                                   uint2* __restrict__ overflow)
 {
-    __shared__ uint32_t s_node[L > 0 ? L * BS : 1];
-    __shared__ float s_t[L > 0 ? L * BS : 1];
+    __shared__ u32x2 s_stack[L > 0 ? L * BS : 1];
     const uint32_t n = counts[bounce];
     const uint32_t lb = xcd_block();
-    const size_t ostride = (size_t)gridDim.x * blockDim.x;
     const size_t oslot = (size_t)lb * blockDim.x + threadIdx.x;
+    if constexpr (W == 4 && L > 0 && !STATS) {
+        LdsStack<L, CAP, BS> st{s_stack, threadIdx.x, overflow, oslot};
+        walk4_stream<false>(
+            st, tnodes, leaves, root, n_leaves, tmin, lb * (BS / 64) + (threadIdx.x >> 6), gridDim.x * (BS / 64), n,
+            [&](uint32_t i, V3& o, V3& d, float& tm) {
+                o = v3(in.ox[i], in.oy[i], in.oz[i]);
+                d = v3(in.dx[i], in.dy[i], in.dz[i]);
+                tm = tmax;
+            },
+            [&](uint32_t i, uint32_t leaf, float t, float ba, float bb) {
+                hit.leaf[i] = leaf;
+                hit.t[i] = t;
+                hit.ba[i] = ba;
+                hit.bb[i] = bb;
+                hit.key[i] = (leaf == NO_HIT) ? 0u : __float_as_uint(leaves[3 * (size_t)leaf + 1].w);
+            });
+        return;
+    }
     uint64_t visits = 0, tests = 0;
     for (uint32_t i = lb * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const V3 o = v3(in.ox[i], in.oy[i], in.oz[i]);
         const V3 d = v3(in.dx[i], in.dy[i], in.dz[i]);
         TraceResult r;
         if constexpr (L > 0) {
-            LdsStack<L, CAP, BS> st{s_node, s_t, threadIdx.x, overflow, ostride, oslot};
+            LdsStack<L, CAP, BS> st{s_stack, threadIdx.x, overflow, oslot};
             r = traverse_w<W, false, STATS>(st, tnodes, leaves, root, n_leaves, o, d, tmin, tmax);
         } else {
             PrivateStack<CAP> st;
@@ -159,11 +175,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(lds_stack_w
                                                    uint32_t* __restrict__ counts, uint32_t bounce, float tmin,
                                                    float tmax, HitBuf hit, uint2* __restrict__ overflow)
 {
-    __shared__ uint32_t s_node[L > 0 ? L * 256 : 1];
-    __shared__ float s_t[L > 0 ? L * 256 : 1];
+    __shared__ u32x2 s_stack[L > 0 ? L * 256 : 1];
     const uint32_t n = counts[bounce];
     const uint32_t lb = xcd_block();
-    const size_t ostride = (size_t)gridDim.x * blockDim.x;
     const size_t oslot = (size_t)lb * blockDim.x + threadIdx.x;
     uint64_t visits = 0, tests = 0;
     for (uint32_t i = lb * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
@@ -176,7 +190,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(lds_stack_w
             wd = v3(in.dx[i], in.dy[i], in.dz[i]);
         };
         if constexpr (L > 0) {
-            LdsStack<L, CAP, 256> st{s_node, s_t, threadIdx.x, overflow, ostride, oslot};
+            LdsStack<L, CAP, 256> st{s_stack, threadIdx.x, overflow, oslot};
             r = two_level_w<W, false, STATS>(st, top4, top_leaves, top_root, n_inst, inst, mesh_nodes, leaves, o, d,
                                              tmin, tmax, ii, world);
         } else {

@@ -110,11 +110,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(lds_stack_w
                                                      const uint32_t* __restrict__ in_slot, HitBuf hit,
                                                      uint2* __restrict__ overflow)
 {
-    __shared__ uint32_t s_node[L > 0 ? L * 256 : 1];
-    __shared__ float s_t[L > 0 ? L * 256 : 1];
+    __shared__ u32x2 s_stack[L > 0 ? L * 256 : 1];
     const uint32_t n = hdr->n_total;
     const uint32_t lb = xcd_block();
-    const size_t ostride = (size_t)gridDim.x * blockDim.x;
     const size_t oslot = (size_t)lb * blockDim.x + threadIdx.x;
     for (uint32_t i = lb * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const SlotDev& sd = slots[in_slot[i]];
@@ -129,7 +127,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(lds_stack_w
         const uint32_t root = (W == 4) ? sd.root4 : sd.root;
         TraceResult r;
         if constexpr (L > 0) {
-            LdsStack<L, CAP, 256> st{s_node, s_t, threadIdx.x, overflow, ostride, oslot};
+            LdsStack<L, CAP, 256> st{s_stack, threadIdx.x, overflow, oslot};
             r = traverse_w<W, false, false>(st, nodes, leaves, root, sd.n_leaves, o, d, tmin, tmax);
         } else {
             PrivateStack<CAP> st;
@@ -152,11 +150,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(lds_stack_w
     const uint32_t* __restrict__ in_slot, HitBuf hit, uint2* __restrict__ overflow)
 {
     constexpr int CAP = 128;
-    __shared__ uint32_t s_node[L > 0 ? L * 256 : 1];
-    __shared__ float s_t[L > 0 ? L * 256 : 1];
+    __shared__ u32x2 s_stack[L > 0 ? L * 256 : 1];
     const uint32_t n = hdr->n_total;
     const uint32_t lb = xcd_block();
-    const size_t ostride = (size_t)gridDim.x * blockDim.x;
     const size_t oslot = (size_t)lb * blockDim.x + threadIdx.x;
     for (uint32_t i = lb * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const SlotDev& sd = slots[in_slot[i]];
@@ -174,7 +170,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(lds_stack_w
         TraceResult r;
         uint32_t ii;
         if constexpr (L > 0) {
-            LdsStack<L, CAP, 256> st{s_node, s_t, threadIdx.x, overflow, ostride, oslot};
+            LdsStack<L, CAP, 256> st{s_stack, threadIdx.x, overflow, oslot};
             r = two_level_w<W, false, false>(st, sd.nodes4, sd.top_leaves, sd.root4, sd.n_leaves, sd.inst, mesh_nodes,
                                              sd.q.leaves, o, d, tmin, tmax, ii, world);
         } else {

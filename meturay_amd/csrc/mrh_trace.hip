@@ -17,18 +17,38 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(lds_stack_w
                                                float* __restrict__ out_bary, uint32_t* __restrict__ stats,
                                                uint2* __restrict__ overflow)
 {
-    __shared__ uint32_t s_node[L > 0 ? L * 256 : 1];
-    __shared__ float s_t[L > 0 ? L * 256 : 1];
+    __shared__ u32x2 s_stack[L > 0 ? L * 256 : 1];
     const uint32_t lb = xcd_block();
-    const size_t ostride = (size_t)gridDim.x * blockDim.x;
     const size_t oslot = (size_t)lb * blockDim.x + threadIdx.x;
+    if constexpr (W == 4 && L > 0 && !STATS) {
+        LdsStack<L, CAP, 256> st{s_stack, threadIdx.x, overflow, oslot};
+        walk4_stream<ANY>(
+            st, tnodes, leaves, root, n_leaves, tmin, lb * 4 + (threadIdx.x >> 6), gridDim.x * 4, n,
+            [&](uint32_t i, V3& o, V3& d, float& tmax) {
+                o = v3(rays[i], rays[(size_t)pitch + i], rays[2 * (size_t)pitch + i]);
+                d = v3(rays[3 * (size_t)pitch + i], rays[4 * (size_t)pitch + i], rays[5 * (size_t)pitch + i]);
+                tmax = rays[6 * (size_t)pitch + i];
+            },
+            [&](uint32_t i, uint32_t leaf, float t, float ba, float bb) {
+                const bool hit = leaf != NO_HIT;
+                if (ANY) {
+                    out_prim[i] = hit ? 1u : 0u;
+                } else {
+                    out_prim[i] = hit ? __float_as_uint(leaves[3 * (size_t)leaf].w) : NO_HIT;
+                    out_t[i] = hit ? t : 0.0f;
+                    out_bary[i] = hit ? ba : 0.0f;
+                    out_bary[(size_t)n + i] = hit ? bb : 0.0f;
+                }
+            });
+        return;
+    }
     for (uint32_t i = lb * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const V3 o = v3(rays[i], rays[(size_t)pitch + i], rays[2 * (size_t)pitch + i]);
         const V3 d = v3(rays[3 * (size_t)pitch + i], rays[4 * (size_t)pitch + i], rays[5 * (size_t)pitch + i]);
         const float tmax = rays[6 * (size_t)pitch + i];
         TraceResult r;
         if constexpr (L > 0) {
-            LdsStack<L, CAP, 256> st{s_node, s_t, threadIdx.x, overflow, ostride, oslot};
+            LdsStack<L, CAP, 256> st{s_stack, threadIdx.x, overflow, oslot};
             r = traverse_w<W, ANY, STATS>(st, tnodes, leaves, root, n_leaves, o, d, tmin, tmax);
         } else {
             PrivateStack<CAP> st;

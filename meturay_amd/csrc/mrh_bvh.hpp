@@ -572,23 +572,23 @@ struct Walk4 {
         leaf = NO_HIT;
         ba = bb = 0.0f;
     }
-    // a leaf in `next` moves to a free `pend` (NO_HIT and out-of-range codes
-    // are no leaf)
-    __device__ __forceinline__ void stash(uint32_t n_leaves)
+    // a leaf in `next` moves to a free `pend`; true when `next` is then
+    // neither a node nor a leaf that waits (NO_HIT, or a code out of range)
+    __device__ __forceinline__ bool stash(uint32_t n_leaves)
     {
         const uint32_t li = next ^ LEAF_BIT;
-        const bool put = li < n_leaves && pend == NO_HIT;
+        const bool is_leaf = li < n_leaves, put = is_leaf && pend == NO_HIT;
         pend = put ? li : pend;
         pend_t = put ? next_t : pend_t;
         next = put ? NO_HIT : next;
+        return (put | !is_leaf) & !(next < n_leaves - 1u);
     }
     // at most one pop: a second one in the same step would keep the wave's
     // other lanes waiting for the few that need it
     template <class Stack>
     __device__ __forceinline__ void settle(const Stack& st, uint32_t n_leaves)
     {
-        stash(n_leaves);
-        if (next == NO_HIT && sp > 0) {
+        if (stash(n_leaves) && sp > 0) {
             --sp;
             uint32_t nn;
             st.get(sp, nn, next_t);
@@ -655,17 +655,24 @@ constexpr uint32_t WALK_REFILL = 48;
 // CU's address unit 70 % busy) and by VALU issue (75 %).  Against the
 // one-ray-per-lane loop over traverse4: the frame above 16.5 -> 14.5 ms, the
 // casts 11.0 -> 6.6 ms.
+//
+// tr is the tree of every ray, unless fetch sets another one for its lane
+// (the serving engine's rays each have their own scene); a ray for which
+// fetch returns false is left out.
+struct Tree4 {
+    const float4* nodes;
+    const float4* leaves;
+    uint32_t root, n_leaves;
+    float tmin;
+};
+
 template <bool ANY, class Stack, class Fetch, class Emit>
-__device__ __forceinline__ void walk4_stream(Stack& st, const float4* __restrict__ nodes4,
-                                             const float4* __restrict__ leaves, uint32_t root, uint32_t n_leaves,
-                                             float tmin, uint32_t wave, uint32_t waves, uint32_t n, Fetch&& fetch,
-                                             Emit&& emit)
+__device__ __forceinline__ void walk4_stream(Stack& st, Tree4 tr, uint32_t wave, uint32_t waves, uint32_t n,
+                                             Fetch&& fetch, Emit&& emit)
 {
     uint32_t G = 64u;
     while (G > TRACE_MIN_GROUP && (uint64_t)waves * (G >> 1) >= n) G >>= 1;
     const uint32_t stride = waves * G;
-    const char* nbase = (const char*)nodes4;
-    const uint32_t n_int = n_leaves - 1u;
     uint32_t group = __builtin_amdgcn_readfirstlane(wave) * G, used = 0;   // next rays of the wave
     uint32_t ray = NO_HIT;
     Walk4 w;
@@ -673,18 +680,18 @@ __device__ __forceinline__ void walk4_stream(Stack& st, const float4* __restrict
     for (;;) {
         uint64_t ma;
         for (;;) {
-            w.settle(st, n_leaves);
-            const bool can = w.next < n_int;
+            w.settle(st, tr.n_leaves);
+            const bool can = w.next < tr.n_leaves - 1u;
             const uint64_t mc = __ballot(can), mp = __ballot(w.pend != NO_HIT);
             ma = mc | mp | __ballot(w.sp > 0);
             if ((uint32_t)__popcll(ma) <= 64u - WALK_REFILL && (group < n || !ma)) break;
             if (!mp || 8u * (uint32_t)__popcll(mc) >= 5u * (uint32_t)__popcll(ma)) {
-                if (can) w.next = node4_near_push(st, w.sp, node4_test(nbase, w.next << 7, w.sl, tmin, w.t), w.next_t);
+                if (can) w.next = node4_near_push(st, w.sp, node4_test((const char*)tr.nodes, w.next << 7, w.sl, tr.tmin, w.t), w.next_t);
             } else {
-                if (w.pend != NO_HIT) w.test_leaf<ANY>(leaves, tmin);
+                if (w.pend != NO_HIT) w.test_leaf<ANY>(tr.leaves, tr.tmin);
             }
         }
-        const bool dead = !(w.next < n_int || w.pend != NO_HIT || w.sp > 0);
+        const bool dead = !(w.next < tr.n_leaves - 1u || w.pend != NO_HIT || w.sp > 0);
         if (dead && ray != NO_HIT) {
             emit(ray, w.leaf, w.t, w.ba, w.bb);
             ray = NO_HIT;
@@ -693,11 +700,10 @@ __device__ __forceinline__ void walk4_stream(Stack& st, const float4* __restrict
         if (dead) {
             const uint32_t q = used + rank_below(~ma);
             const uint32_t i = group + q + (q >= G ? stride - G : 0u);
-            if (i < n) {
-                V3 o, d;
-                float tmax;
-                fetch(i, o, d, tmax);
-                w.begin(o, d, tmax, root);
+            V3 o, d;
+            float tmax;
+            if (i < n && fetch(i, o, d, tmax, tr)) {
+                w.begin(o, d, tmax, tr.root);
                 ray = i;
             }
         }
@@ -865,6 +871,150 @@ __device__ __forceinline__ TraceResult traverse_two_level(Stack& st, const float
         }
         if (STATS) r.visits++;
         next = node4_order_push(st, sp, node4_test(tbase, next << 7, sl, tmin, r.t));
+    }
+}
+
+// One lane's state in walk2l_stream: Walk4 over the tree it is in, and the
+// instance whose space the ray is in (cur; NO_HIT: the world).  base is the
+// stack depth at the instance's entry, -1 in the top tree.
+struct Walk2L {
+    Walk4 w;
+    int base;
+    uint32_t cur, n_cur;    // n_cur: leaves of the current tree
+    const float4* nodes;
+    uint32_t leaf_base;     // first leaf record of the instance's mesh
+    uint32_t hit_inst;
+    __device__ __forceinline__ void begin(V3 o, V3 d, float tmax, const float4* top4, uint32_t root, uint32_t n_inst)
+    {
+        w.begin(o, d, tmax, root);
+        base = -1;
+        cur = NO_HIT;
+        n_cur = n_inst;
+        nodes = top4;
+        leaf_base = 0;
+        hit_inst = NO_HIT;
+    }
+    // Walk4::settle; a mesh's leaves are all tested before its instance is
+    // left, and an instance (a leaf of the top tree) is never put off
+    template <class Stack>
+    __device__ __forceinline__ void settle(const Stack& st, uint32_t n_inst)
+    {
+        bool empty;
+        if (base >= 0) {
+            empty = w.stash(n_cur);
+            if (empty && w.sp == base && w.pend == NO_HIT) {
+                base = -1;
+                n_cur = n_inst;
+            }
+        } else {
+            empty = !(w.next < n_cur - 1u) && !((w.next ^ LEAF_BIT) < n_cur);
+        }
+        if (empty && w.sp > (base > 0 ? base : 0)) {
+            --w.sp;
+            uint32_t nn;
+            st.get(w.sp, nn, w.next_t);
+            w.next = (w.next_t > w.t) ? NO_HIT : nn;
+            if (base >= 0) w.stash(n_cur);
+        }
+    }
+};
+
+// traverse_two_level4's walk for the rays of a wave, with walk4_stream's
+// turns (leaves put off, refill; equal bits for the same reasons) and a third
+// kind of step, the change of the ray's space: a lane that comes to an
+// instance, or back to a node of the top tree, reloads the world ray, takes
+// it to the instance's space and forms its slab constants.  Going from one
+// instance to the next is one such step.  The wave takes the step that most
+// lanes wait for once fewer than 5/8 can test a node.
+template <class Stack, class Fetch, class Emit>
+__device__ __forceinline__ void walk2l_stream(Stack& st, const float4* __restrict__ top4,
+                                              const float4* __restrict__ top_leaves, uint32_t top_root,
+                                              uint32_t n_inst, const float4* __restrict__ inst,
+                                              const float4* __restrict__ mesh_nodes,
+                                              const float4* __restrict__ leaves, float tmin, uint32_t wave,
+                                              uint32_t waves, uint32_t n, Fetch&& fetch, Emit&& emit)
+{
+    uint32_t G = 64u;
+    while (G > TRACE_MIN_GROUP && (uint64_t)waves * (G >> 1) >= n) G >>= 1;
+    const uint32_t stride = waves * G;
+    uint32_t group = __builtin_amdgcn_readfirstlane(wave) * G, used = 0;
+    uint32_t ray = NO_HIT;
+    Walk2L s;
+    s.begin(v3(0.0f, 0.0f, 0.0f), v3(0.0f, 0.0f, 0.0f), 0.0f, top4, NO_HIT, n_inst);
+    for (;;) {
+        uint64_t ma;
+        bool can, swap;
+        for (;;) {
+            s.settle(st, n_inst);
+            const bool node = s.w.next < s.n_cur - 1u, top = s.base < 0, local = s.cur != NO_HIT;
+            const bool entry = top && (s.w.next ^ LEAF_BIT) < n_inst;
+            can = node && !(top && local);
+            swap = entry || (node && top && local);
+            const uint64_t mc = __ballot(can), mp = __ballot(s.w.pend != NO_HIT), ms = __ballot(swap);
+            ma = mc | mp | ms | __ballot(s.w.sp > 0);
+            if ((uint32_t)__popcll(ma) <= 64u - WALK_REFILL && (group < n || !ma)) break;
+            if (!(mp | ms) || 8u * (uint32_t)__popcll(mc) >= 5u * (uint32_t)__popcll(ma)) {
+                if (can)
+                    s.w.next = node4_near_push(st, s.w.sp,
+                                               node4_test((const char*)s.nodes, s.w.next << 7, s.w.sl, tmin, s.w.t),
+                                               s.w.next_t);
+            } else if (__popcll(mp) >= __popcll(ms)) {
+                if (s.w.pend != NO_HIT) {
+                    const float t0 = s.w.t;
+                    s.w.test_leaf<false>(leaves + 3 * (size_t)s.leaf_base, tmin);
+                    const bool hit = s.w.t < t0;
+                    s.w.leaf = hit ? s.w.leaf + s.leaf_base : s.w.leaf;
+                    s.hit_inst = hit ? s.cur : s.hit_inst;
+                }
+            } else if (swap) {
+                float tmax;
+                fetch(ray, s.w.o, s.w.d, tmax);
+                s.cur = NO_HIT;
+                s.nodes = top4;
+                if (entry) {
+                    const uint32_t ii = __float_as_uint(top_leaves[3 * (size_t)(s.w.next ^ LEAF_BIT)].w);
+                    s.w.next = NO_HIT;
+                    if (ii < n_inst) {   // always, on a well-formed tree
+                        const float4* rec = inst + INST_F4 * (size_t)ii;
+                        const float4 w0 = rec[0], w1 = rec[1], w2 = rec[2];
+                        const float4 m6 = rec[6], m7 = rec[7];
+                        const V3 lo = xf_point(w0, w1, w2, s.w.o);
+                        s.w.d = xf_dir(w0, w1, w2, s.w.d);
+                        s.w.o = lo;
+                        s.base = s.w.sp;
+                        s.cur = ii;
+                        s.n_cur = __float_as_uint(m7.w);
+                        s.nodes = mesh_nodes + 8 * (size_t)__float_as_uint(m7.x);
+                        s.leaf_base = __float_as_uint(m6.z);
+                        s.w.next = __float_as_uint(m7.y);
+                        s.w.next_t = -INFINITY;
+                    }
+                }
+                s.w.sl = make_slab(s.w.o, s.w.d);
+            }
+        }
+        const bool dead = !(can || swap || s.w.pend != NO_HIT || s.w.sp > 0);
+        if (dead && ray != NO_HIT) {
+            emit(ray, s.w.leaf, s.hit_inst, s.w.t, s.w.ba, s.w.bb);
+            ray = NO_HIT;
+        }
+        if (group >= n) break;
+        if (dead) {
+            const uint32_t q = used + rank_below(~ma);
+            const uint32_t i = group + q + (q >= G ? stride - G : 0u);
+            if (i < n) {
+                V3 o, d;
+                float tmax;
+                fetch(i, o, d, tmax);
+                s.begin(o, d, tmax, top4, top_root, n_inst);
+                ray = i;
+            }
+        }
+        used += (uint32_t)__popcll(~ma);
+        if (used >= G) {
+            used -= G;
+            group += stride;
+        }
     }
 }
 

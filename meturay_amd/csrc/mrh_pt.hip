@@ -63,11 +63,12 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(lds_stack_wa
     if constexpr (W == 4 && L > 0 && !STATS) {
         LdsStack<L, CAP, BS> st{s_stack, threadIdx.x, overflow, oslot};
         walk4_stream<false>(
-            st, tnodes, leaves, root, n_leaves, tmin, lb * (BS / 64) + (threadIdx.x >> 6), gridDim.x * (BS / 64), n,
-            [&](uint32_t i, V3& o, V3& d, float& tm) {
+            st, Tree4{tnodes, leaves, root, n_leaves, tmin}, lb * (BS / 64) + (threadIdx.x >> 6), gridDim.x * (BS / 64), n,
+            [&](uint32_t i, V3& o, V3& d, float& tm, Tree4&) {
                 o = v3(in.ox[i], in.oy[i], in.oz[i]);
                 d = v3(in.dx[i], in.dy[i], in.dz[i]);
                 tm = tmax;
+                return true;
             },
             [&](uint32_t i, uint32_t leaf, float t, float ba, float bb) {
                 hit.leaf[i] = leaf;
@@ -162,10 +163,12 @@ int32_t launch_trace_pt(mrh_context* ctx, uint32_t grid, const mrh_lbvh* b, cons
 }
 
 // Two-level scenes: the top tree over the instances, then the hit mesh's
-// tree in local space (traverse_two_level); writes the instance too, and the
-// instance's HitKey override where it has one.  Five waves per SIMD: the
-// walk needs 90 registers; capped at 80 (six waves) it spills and runs 3 %
-// slower, at 72 or 64 it spills far more (1.4x and 2.9x the frame time).
+// tree in local space (walk2l_stream; traverse_two_level for the other tree
+// widths and the counting variant); writes the instance too, and the
+// instance's HitKey override where it has one.  Five waves per SIMD: the walk
+// needs 89 registers.  1280x720 frame with NEE over 4096 instances: 8.48 ms
+// with one ray per lane, 6.65 ms with the stream (7.14 ms at six waves, which
+// spill).
 template <int W, int CAP, bool STATS, int L>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(lds_stack_waves(L, 256, 5)))) void k_trace_pt2(const float4* __restrict__ top4,
                                                    const float4* __restrict__ top_leaves, uint32_t top_root,
@@ -179,6 +182,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(lds_stack_w
     const uint32_t n = counts[bounce];
     const uint32_t lb = xcd_block();
     const size_t oslot = (size_t)lb * blockDim.x + threadIdx.x;
+    if constexpr (W == 4 && L > 0 && !STATS) {
+        LdsStack<L, CAP, 256> st{s_stack, threadIdx.x, overflow, oslot};
+        walk2l_stream(
+            st, top4, top_leaves, top_root, n_inst, inst, mesh_nodes, leaves, tmin, lb * 4 + (threadIdx.x >> 6),
+            gridDim.x * 4, n,
+            [&](uint32_t i, V3& o, V3& d, float& tm) {
+                o = v3(in.ox[i], in.oy[i], in.oz[i]);
+                d = v3(in.dx[i], in.dy[i], in.dz[i]);
+                tm = tmax;
+            },
+            [&](uint32_t i, uint32_t leaf, uint32_t ii, float t, float ba, float bb) {
+                hit.leaf[i] = leaf;
+                hit.t[i] = t;
+                hit.ba[i] = ba;
+                hit.bb[i] = bb;
+                hit.inst[i] = ii;
+                uint32_t key = 0u;
+                if (leaf != NO_HIT) {
+                    const uint32_t ko = __float_as_uint(inst[INST_F4 * (size_t)ii + 6].y);
+                    key = ko ? ko : __float_as_uint(leaves[3 * (size_t)leaf + 1].w);
+                }
+                hit.key[i] = key;
+            });
+        return;
+    }
     uint64_t visits = 0, tests = 0;
     for (uint32_t i = lb * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const V3 o = v3(in.ox[i], in.oy[i], in.oz[i]);

@@ -23,11 +23,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(lds_stack_w
     if constexpr (W == 4 && L > 0 && !STATS) {
         LdsStack<L, CAP, 256> st{s_stack, threadIdx.x, overflow, oslot};
         walk4_stream<ANY>(
-            st, tnodes, leaves, root, n_leaves, tmin, lb * 4 + (threadIdx.x >> 6), gridDim.x * 4, n,
-            [&](uint32_t i, V3& o, V3& d, float& tmax) {
+            st, Tree4{tnodes, leaves, root, n_leaves, tmin}, lb * 4 + (threadIdx.x >> 6), gridDim.x * 4, n,
+            [&](uint32_t i, V3& o, V3& d, float& tmax, Tree4&) {
                 o = v3(rays[i], rays[(size_t)pitch + i], rays[2 * (size_t)pitch + i]);
                 d = v3(rays[3 * (size_t)pitch + i], rays[4 * (size_t)pitch + i], rays[5 * (size_t)pitch + i]);
                 tmax = rays[6 * (size_t)pitch + i];
+                return true;
             },
             [&](uint32_t i, uint32_t leaf, float t, float ba, float bb) {
                 const bool hit = leaf != NO_HIT;

@@ -59,3 +59,22 @@ def test_stream_walk_equals_oracle(ctx, oracle, n, m, lds):
     assert t.cpu().numpy().tobytes() == rt.tobytes()
     assert bary.cpu().numpy().tobytes() == rb.tobytes()
     assert np.array_equal(anyh.cpu().numpy() != 0, rp != 0xFFFFFFFF)
+
+
+@pytest.mark.parametrize("two_level", [0, 1])
+@pytest.mark.parametrize("w,h", [(5, 3), (17, 31), (200, 111)])
+def test_frame_equals_counting_walk(ctx, w, h, two_level):
+    """A frame traced by the streaming walk (flat and two-level) and by the
+    counting one-ray walk: the same paths, so the same segments and image up
+    to the order of a pixel's adds (S^2 = 4 of them and a path's few
+    emitters: 8 float adds at most)."""
+    sc = N.gen_instanced_sphere_grid(15, 8, 8, 3, 4) if two_level else N.gen_sphere_grid(15, 8, 8, 3)
+    scene = N.Scene(ctx, sc)
+    img = [torch.zeros(h, w, 3, device="cuda") for _ in range(2)]
+    torch.cuda.synchronize()
+    st = [scene.render(img[k], w, h, 2, 9, 3, 5, nee=1, mis=1, count_traversal=bool(k)) for k in range(2)]
+    scene.close()
+    assert st[0].segments == st[1].segments
+    assert list(st[0].bounce_rays) == list(st[1].bounce_rays)
+    a, b = img[0].cpu().numpy(), img[1].cpu().numpy()
+    assert np.all(np.abs(a - b) <= 8 * 2.0 ** -24 * np.maximum(np.abs(a), np.abs(b)).max())

@@ -145,6 +145,7 @@ int32_t mrh_context_destroy(mrh_context* ctx)
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
     if (ctx->guide_svo) mrh_svo_destroy(ctx->guide_svo);
+    if (ctx->wfpg_svo) mrh_svo_destroy(ctx->wfpg_svo);
     for (int i = 0; i < SLOT_COUNT; i++)
         if (ctx->slot_ptr[i]) (void)hipFree(ctx->slot_ptr[i]);
     for (auto& p : ctx->pending) { (void)hipEventDestroy(p.a); (void)hipEventDestroy(p.b); }

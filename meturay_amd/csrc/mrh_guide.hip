@@ -22,7 +22,7 @@
 
 struct mrh_svo {
     mrh_context* ctx = nullptr;
-    uint32_t depth = 0, nodes = 0, cap = 0;
+    uint32_t depth = 0, nodes = 0, cap = 0, rad_cap = 0;   // rad_cap: nodes of the radiance arrays
     uint32_t lvl_count[11] = {}, lvl_off[12] = {};
     float cube[4] = {0, 0, 0, 1};   // lo xyz, size
     uint32_t* codes = nullptr;       // [cap] level code of each node
@@ -1038,32 +1038,39 @@ SvoView svo_view(const mrh_svo* s)
     return v;
 }
 
-static int32_t svo_reserve(mrh_svo* s, uint32_t nodes)
+static int32_t svo_reserve(mrh_svo* s, uint32_t nodes, bool radiance)
 {
     mrh_context* ctx = s->ctx;
-    if (nodes <= s->cap) return MRH_OK;
-    (void)hipStreamSynchronize(ctx->stream);
-    void* ptrs[] = {s->codes, s->first_child, s->child_mask, s->parent, s->sum, s->acc, s->cnt, s->radiance,
-                    s->node_count, s->pack};
-    for (void* p : ptrs) (void)hipFree(p);
-    s->codes = s->first_child = s->child_mask = s->parent = s->node_count = nullptr;
-    s->pack = nullptr;
-    s->sum = s->radiance = nullptr;
-    s->acc = nullptr;
-    s->cnt = nullptr;
-    s->cap = 0;
     const uint32_t cap = nodes + nodes / 4 + 64;
-    MRH_TRY(dmalloc(ctx, (void**)&s->codes, (size_t)cap * 4));
-    MRH_TRY(dmalloc(ctx, (void**)&s->first_child, (size_t)cap * 4));
-    MRH_TRY(dmalloc(ctx, (void**)&s->child_mask, (size_t)cap * 4));
-    MRH_TRY(dmalloc(ctx, (void**)&s->parent, (size_t)cap * 4));
-    MRH_TRY(dmalloc(ctx, (void**)&s->sum, (size_t)cap * GUIDE_BINS * 4));
-    MRH_TRY(dmalloc(ctx, (void**)&s->acc, (size_t)cap * GUIDE_BINS * 8));
-    MRH_TRY(dmalloc(ctx, (void**)&s->cnt, (size_t)cap * GUIDE_BINS * 4));
-    MRH_TRY(dmalloc(ctx, (void**)&s->radiance, (size_t)cap * GUIDE_BINS * 4));
-    MRH_TRY(dmalloc(ctx, (void**)&s->node_count, (size_t)cap * 4));
-    MRH_TRY(dmalloc(ctx, (void**)&s->pack, (size_t)cap * 16));
-    s->cap = cap;
+    if (nodes > s->cap) {
+        (void)hipStreamSynchronize(ctx->stream);
+        void* ptrs[] = {s->codes, s->first_child, s->child_mask, s->parent, s->pack};
+        for (void* p : ptrs) (void)hipFree(p);
+        s->codes = s->first_child = s->child_mask = s->parent = nullptr;
+        s->pack = nullptr;
+        s->cap = 0;
+        MRH_TRY(dmalloc(ctx, (void**)&s->codes, (size_t)cap * 4));
+        MRH_TRY(dmalloc(ctx, (void**)&s->first_child, (size_t)cap * 4));
+        MRH_TRY(dmalloc(ctx, (void**)&s->child_mask, (size_t)cap * 4));
+        MRH_TRY(dmalloc(ctx, (void**)&s->parent, (size_t)cap * 4));
+        MRH_TRY(dmalloc(ctx, (void**)&s->pack, (size_t)cap * 16));
+        s->cap = cap;
+    }
+    if (radiance && nodes > s->rad_cap) {
+        (void)hipStreamSynchronize(ctx->stream);
+        void* ptrs[] = {s->sum, s->acc, s->cnt, s->radiance, s->node_count};
+        for (void* p : ptrs) (void)hipFree(p);
+        s->sum = s->radiance = nullptr;
+        s->acc = nullptr;
+        s->cnt = s->node_count = nullptr;
+        s->rad_cap = 0;
+        MRH_TRY(dmalloc(ctx, (void**)&s->sum, (size_t)cap * GUIDE_BINS * 4));
+        MRH_TRY(dmalloc(ctx, (void**)&s->acc, (size_t)cap * GUIDE_BINS * 8));
+        MRH_TRY(dmalloc(ctx, (void**)&s->cnt, (size_t)cap * GUIDE_BINS * 4));
+        MRH_TRY(dmalloc(ctx, (void**)&s->radiance, (size_t)cap * GUIDE_BINS * 4));
+        MRH_TRY(dmalloc(ctx, (void**)&s->node_count, (size_t)cap * 4));
+        s->rad_cap = cap;
+    }
     return MRH_OK;
 }
 
@@ -1096,7 +1103,7 @@ static int32_t grow(mrh_context* ctx, void** p, size_t* have, size_t want)
 // and the parent index of the level below; then links, lookup records and
 // fresh radiance.
 int32_t svo_build(mrh_context* ctx, mrh_svo* s, const uint32_t* d_codes, uint32_t n, const float cube[4],
-                  uint32_t depth, bool filtered)
+                  uint32_t depth, SvoContent content)
 {
     if (depth < 1 || depth > 10) return fail(ctx, MRH_ERR_INVALID, "svo depth must be in [1, 10]");
     if (n == 0) return fail(ctx, MRH_ERR_INVALID, "svo build: no points");
@@ -1152,7 +1159,7 @@ int32_t svo_build(mrh_context* ctx, mrh_svo* s, const uint32_t* d_codes, uint32_
     for (int l = (int)depth - 1; l >= 0; l--)
         MRH_TRY(unique_runs(ctx, lvl_codes[l + 1], s->lvl_count[l + 1], 3, lvl_codes[l], lvl_parent[l + 1], flags,
                             pos, tmp));
-    MRH_TRY(svo_reserve(s, s->nodes));
+    MRH_TRY(svo_reserve(s, s->nodes, content != SVO_GEOMETRY));
     for (uint32_t l = 0; l <= depth; l++) {
         const uint32_t c = s->lvl_count[l];
         MRH_TRY(launch(ctx, "svo_link", dim3(stride_grid(ctx, c, 256)), dim3(256), 0, k_svo_link,
@@ -1162,10 +1169,11 @@ int32_t svo_build(mrh_context* ctx, mrh_svo* s, const uint32_t* d_codes, uint32_
     MRH_TRY(launch(ctx, "svo_pack", dim3(stride_grid(ctx, s->nodes, 256)), dim3(256), 0, k_svo_pack, s->nodes,
                    (const uint32_t*)s->first_child, (const uint32_t*)s->child_mask, (const uint32_t*)nullptr,
                    s->pack));
+    if (content == SVO_GEOMETRY) return MRH_OK;
     // fresh radiance
     MRH_TRY(fill_u32(ctx, (uint32_t*)s->acc, 0u, (size_t)s->nodes * GUIDE_BINS * 2));
     MRH_TRY(fill_u32(ctx, s->cnt, 0u, (size_t)s->nodes * GUIDE_BINS));
-    if (filtered) return MRH_OK;
+    if (content == SVO_FILTERED_LATER) return MRH_OK;
     MRH_TRY(fill_u32(ctx, (uint32_t*)s->sum, 0u, (size_t)s->nodes * GUIDE_BINS));
     uint32_t eps_bits;
     std::memcpy(&eps_bits, &GUIDE_EPS, 4);
@@ -1433,16 +1441,12 @@ int32_t svo_bin_rays(mrh_context* ctx, mrh_svo* s, const uint32_t* codes, uint32
 }
 
 }  // namespace
-}  // namespace mrh
 
-using namespace mrh;
-
-extern "C" {
-
-int32_t mrh_svo_voxelize(mrh_context* ctx, const float* d_tris, uint32_t n, const float cube[4], uint32_t depth,
-                         uint32_t* d_codes, uint32_t* d_prims, uint32_t capacity, uint32_t* out_count)
+// SLOT_VOXEL: a 64-bit total, counts[n + 1] (scanned in place into offsets
+// by the write half), scan scratch
+int32_t svo_voxelize_count(mrh_context* ctx, const float* d_tris, uint32_t n, const float cube[4], uint32_t depth,
+                           uint32_t* out_count)
 {
-    if (!ctx || !cube || !out_count) return MRH_ERR_INVALID;
     *out_count = 0;
     if (depth < 1 || depth > 10) return fail(ctx, MRH_ERR_INVALID, "mrh_svo_voxelize: depth must be in [1, 10]");
     for (int a = 0; a < 4; a++)
@@ -1451,13 +1455,11 @@ int32_t mrh_svo_voxelize(mrh_context* ctx, const float* d_tris, uint32_t n, cons
     if (n == 0) return MRH_OK;
     if (!d_tris) return fail(ctx, MRH_ERR_INVALID, "mrh_svo_voxelize: null triangles");
     if (n >= (1u << 30)) return fail(ctx, MRH_ERR_INVALID, "mrh_svo_voxelize: at most 2^30 - 1 triangles");
-    // counts[n + 1] (scanned in place into offsets), scan scratch, a 64-bit total
     const size_t words = 2 + (size_t)n + 1 + scan_tmp_words(n + 1);
     void* mem = nullptr;
     MRH_TRY(scratch(ctx, SLOT_VOXEL, words * 4, &mem));
     unsigned long long* total = (unsigned long long*)mem;
     uint32_t* counts = (uint32_t*)mem + 2;
-    uint32_t* tmp = counts + n + 1;
     const float4 c4 = make_float4(cube[0], cube[1], cube[2], cube[3]);
     const uint32_t grid = (uint32_t)std::min<uint64_t>(div_up(n, 4), (uint64_t)ctx->num_cus * 8u);
     MRH_TRY(fill_u32(ctx, (uint32_t*)mem, 0u, 2));
@@ -1470,10 +1472,33 @@ int32_t mrh_svo_voxelize(mrh_context* ctx, const float* d_tris, uint32_t n, cons
     if (h_total > 0xFFFFFFFFull)
         return fail(ctx, MRH_ERR_INVALID, "mrh_svo_voxelize: %llu voxel records exceed 2^32 - 1", h_total);
     *out_count = (uint32_t)h_total;
-    if (!d_codes || h_total > capacity || h_total == 0) return MRH_OK;   // a size query
-    MRH_TRY(scan_exclusive(ctx, counts, counts, n + 1, tmp));
-    return launch(ctx, "voxelize", dim3(grid), dim3(256), 0, k_voxelize, d_tris, n, c4, depth,
-                  (const uint32_t*)counts, d_codes, d_prims, (unsigned long long*)nullptr);
+    return MRH_OK;
+}
+
+int32_t svo_voxelize_write(mrh_context* ctx, const float* d_tris, uint32_t n, const float cube[4], uint32_t depth,
+                           uint32_t* d_codes, uint32_t* d_prims)
+{
+    uint32_t* counts = (uint32_t*)ctx->slot_ptr[SLOT_VOXEL] + 2;
+    MRH_TRY(scan_exclusive(ctx, counts, counts, n + 1, counts + n + 1));
+    const uint32_t grid = (uint32_t)std::min<uint64_t>(div_up(n, 4), (uint64_t)ctx->num_cus * 8u);
+    return launch(ctx, "voxelize", dim3(grid), dim3(256), 0, k_voxelize, d_tris, n,
+                  make_float4(cube[0], cube[1], cube[2], cube[3]), depth, (const uint32_t*)counts, d_codes, d_prims,
+                  (unsigned long long*)nullptr);
+}
+
+}  // namespace mrh
+
+using namespace mrh;
+
+extern "C" {
+
+int32_t mrh_svo_voxelize(mrh_context* ctx, const float* d_tris, uint32_t n, const float cube[4], uint32_t depth,
+                         uint32_t* d_codes, uint32_t* d_prims, uint32_t capacity, uint32_t* out_count)
+{
+    if (!ctx || !cube || !out_count) return MRH_ERR_INVALID;
+    MRH_TRY(svo_voxelize_count(ctx, d_tris, n, cube, depth, out_count));
+    if (!d_codes || *out_count > capacity || *out_count == 0) return MRH_OK;   // a size query
+    return svo_voxelize_write(ctx, d_tris, n, cube, depth, d_codes, d_prims);
 }
 
 static ConeTree cone_tree(const mrh_svo* s)

@@ -295,11 +295,21 @@ __device__ __forceinline__ float guide_pdf(const SvoView& s, uint32_t node, V3 n
 SvoView svo_view(const mrh_svo* s);
 int32_t svo_codes(mrh_context* ctx, const float* d_points, uint32_t n, uint32_t pitch, const float cube[4],
                   uint32_t depth, uint32_t* d_codes);
-// filtered = true: a splat and a filter follow, which rewrite the means,
+// SVO_FILTERED_LATER: a splat and a filter follow, which rewrite the means,
 // the filtered radiance and the node counts, so only the splat
-// accumulators are cleared
+// accumulators are cleared.  SVO_GEOMETRY: nodes and links only, for trees
+// whose radiance lives elsewhere (the field-traced guide's payload); neither
+// splat, filter nor sampled after.
+enum SvoContent { SVO_FRESH, SVO_FILTERED_LATER, SVO_GEOMETRY };
 int32_t svo_build(mrh_context* ctx, mrh_svo* s, const uint32_t* d_codes, uint32_t n, const float cube[4],
-                  uint32_t depth, bool filtered = false);
+                  uint32_t depth, SvoContent content = SVO_FRESH);
+// mrh_svo_voxelize in its two halves: the record count (the per-triangle
+// counts stay in SLOT_VOXEL), then the records, before anything else uses
+// that slot.
+int32_t svo_voxelize_count(mrh_context* ctx, const float* d_tris, uint32_t n, const float cube[4], uint32_t depth,
+                           uint32_t* out_count);
+int32_t svo_voxelize_write(mrh_context* ctx, const float* d_tris, uint32_t n, const float cube[4], uint32_t depth,
+                           uint32_t* d_codes, uint32_t* d_prims);
 int32_t svo_splat(mrh_context* ctx, mrh_svo* s, const uint32_t* codes, const uint32_t* bins, const float* values,
                   uint32_t n);
 int32_t svo_filter(mrh_context* ctx, mrh_svo* s);

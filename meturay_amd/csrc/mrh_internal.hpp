@@ -32,6 +32,12 @@ enum MrhSlot : int {
     SLOT_SAMPLES,
     SLOT_BOUNDS_PART,
     SLOT_VOXEL,
+    SLOT_WFPG_TRIS,    // field-traced guided renders: triangles, voxel records,
+    SLOT_WFPG_VOXELS,  // node payload, per-ray arrays, path vertices and the
+    SLOT_WFPG_NODES,   // bins of a bounce
+    SLOT_WFPG_RAYS,
+    SLOT_WFPG_VERTS,
+    SLOT_WFPG_BINS,
     SLOT_COUNT
 };
 
@@ -70,6 +76,8 @@ struct mrh_context {
     uint64_t fail_alloc_after = 0;
     // octree reused by guided renders that do not bring their own
     struct mrh_svo* guide_svo = nullptr;
+    // voxel octree reused by field-traced guided renders
+    struct mrh_svo* wfpg_svo = nullptr;
     // this device's fixed partition workspace (mrh_partition_by_key_noalloc);
     // null when its address lookup failed (the reason in noalloc_err)
     void* noalloc_scratch = nullptr;

@@ -3,7 +3,8 @@
 //
 // One histogram kernel reads the keys once and counts every digit pass;
 // a one-block scan turns the counts into global digit bases; then each pass
-// is a single kernel: a tile of 4096 keys is ranked in LDS with wave64
+// is a single kernel (a sort that fits one tile runs all its passes in one
+// block, k_sort_tile): a tile of 4096 keys is ranked in LDS with wave64
 // ballots (one ballot per digit bit gives each lane the set of lanes holding
 // the same digit), the tile's digit counts are published and the tile looks
 // back over its predecessors' published counts (decoupled look-back) to find
@@ -15,11 +16,16 @@
 namespace mrh {
 namespace {
 
-constexpr int SORT_THREADS = 256;
+// A tile is ranked by 16 waves of 4 x 64 keys: the ranking of one wave is a
+// serial chain (ballots and an LDS counter per 64 keys), and with 4 waves of
+// 16 x 64 keys that chain was most of a pass: a single tile 13.2 -> 4 us, a
+// pass over 1 M 32-bit keys 26.3 -> 16.3 us, over 2 M 32.8 -> 23.4 us.
+constexpr int SORT_THREADS = 1024;
 constexpr int SORT_WAVES = SORT_THREADS / 64;
-constexpr int SORT_ITEMS = 16;
+constexpr int SORT_ITEMS = 4;
 constexpr int SORT_TILE = SORT_THREADS * SORT_ITEMS;   // 4096
 constexpr int MAX_PASSES = 8;
+constexpr int LOOKBACK = 4;
 constexpr uint32_t FLAG_AGG = 1u << 30;
 constexpr uint32_t FLAG_PREFIX = 2u << 30;
 constexpr uint32_t COUNT_MASK = (1u << 30) - 1u;
@@ -44,8 +50,13 @@ struct PassDesc {
     uint32_t part_shift, part_mask, part_flip, part_on;
 };
 
+// 8192 keys a block: half the blocks, and so global atomics on the counters, of
+// 4096-key blocks (2 M keys, one pass: 10.2 us against 12.9; 1 M keys, four
+// passes: 8.2 against 13.1; 16384 keys a block leave CUs idle: 14.8 and 11.0)
+constexpr uint32_t HIST_THREADS = 1024, HIST_KEYS = 8, HIST_CHUNK = HIST_KEYS * HIST_THREADS;
+
 template <class KeyT>
-__global__ __launch_bounds__(256) void k_sort_hist(const KeyT* __restrict__ keys, uint32_t n_max,
+__global__ __launch_bounds__(HIST_THREADS) void k_sort_hist(const KeyT* __restrict__ keys, uint32_t n_max,
                                                    const uint32_t* __restrict__ n_dev, PassDesc pd,
                                                    uint32_t* __restrict__ meta)
 {
@@ -55,11 +66,20 @@ __global__ __launch_bounds__(256) void k_sort_hist(const KeyT* __restrict__ keys
     for (uint32_t i = threadIdx.x; i < 256; i += blockDim.x) s_part[i] = 0;
     __syncthreads();
     const uint32_t n = n_dev ? *n_dev : n_max;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        KeyT k = keys[i];
-        for (uint32_t p = 0; p < pd.passes; p++)
-            atomicAdd(&s_hist[p][digit_of(k, pd.shift[p], pd.mask[p], pd.flip[p])], 1u);
-        if (pd.part_on) atomicAdd(&s_part[digit_of(k, pd.part_shift, pd.part_mask, pd.part_flip)], 1u);
+    for (uint32_t base = blockIdx.x * HIST_CHUNK; base < n; base += gridDim.x * HIST_CHUNK) {
+        KeyT k[HIST_KEYS];
+#pragma unroll
+        for (uint32_t j = 0; j < HIST_KEYS; j++) {
+            const uint32_t i = base + j * HIST_THREADS + threadIdx.x;
+            k[j] = (i < n) ? keys[i] : (KeyT)0;
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < HIST_KEYS; j++) {
+            if (base + j * HIST_THREADS + threadIdx.x >= n) break;
+            for (uint32_t p = 0; p < pd.passes; p++)
+                atomicAdd(&s_hist[p][digit_of(k[j], pd.shift[p], pd.mask[p], pd.flip[p])], 1u);
+            if (pd.part_on) atomicAdd(&s_part[digit_of(k[j], pd.part_shift, pd.part_mask, pd.part_flip)], 1u);
+        }
     }
     __syncthreads();
     for (uint32_t i = threadIdx.x; i < pd.passes * 256; i += blockDim.x) {
@@ -110,111 +130,233 @@ __global__ __launch_bounds__(256) void k_sort_scan(uint32_t* __restrict__ meta, 
 }
 
 template <class KeyT>
+struct SortTile {
+    uint32_t whist[SORT_WAVES][256];
+    uint32_t start[256];
+    uint32_t tmp[8];
+    KeyT keys[SORT_TILE];
+    uint32_t vals[SORT_TILE];
+};
+
+// Stable ranks of a tile's keys by one digit: rk = the key's rank among the
+// equal digits of its wave, t.whist[wave][d] = the offset of the wave's run in
+// digit d, t.start[d] = the digit's first place in the tile; returns digit
+// tid's count (tid < 256).  Key j of a thread is number (wave * ITEMS + j) * 64
+// + lane of the tile; the first tile_n are valid.  The lanes that hold the
+// same digit are found by one ballot per digit bit.
+template <class KeyT>
+__device__ __forceinline__ uint32_t rank_tile(SortTile<KeyT>& t, const KeyT (&k)[SORT_ITEMS], uint32_t tile_n,
+                                              uint32_t shift, uint32_t nbits, uint32_t flip,
+                                              uint32_t (&rk)[SORT_ITEMS], uint32_t (&dg)[SORT_ITEMS])
+{
+    const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const uint32_t mask = (1u << nbits) - 1u;
+    for (uint32_t i = tid; i < SORT_WAVES * 256; i += SORT_THREADS) (&t.whist[0][0])[i] = 0;
+    __syncthreads();
+    const uint64_t lanes_below = (1ull << lane) - 1ull;
+#pragma unroll
+    for (int j = 0; j < SORT_ITEMS; j++) {
+        const bool valid = (wave * SORT_ITEMS + j) * 64 + lane < tile_n;
+        const uint32_t d = digit_of(k[j], shift, mask, flip);
+        uint64_t peers = __ballot(valid);
+        for (uint32_t b = 0; b < nbits; b++) {
+            const uint32_t bit = (d >> b) & 1u;
+            const uint64_t bal = __ballot(bit);
+            peers &= bit ? bal : ~bal;
+        }
+        const uint32_t pre = (uint32_t)__popcll(peers & lanes_below);
+        const uint32_t base = valid ? t.whist[wave][d] : 0u;
+        if (valid && pre == 0) t.whist[wave][d] = base + (uint32_t)__popcll(peers);
+        rk[j] = base + pre;
+        dg[j] = valid ? d : 0xFFFFFFFFu;
+    }
+    __syncthreads();
+    uint32_t count = 0;
+    if (tid < 256) {
+#pragma unroll
+        for (int w = 0; w < SORT_WAVES; w++) {
+            const uint32_t c = t.whist[w][tid];
+            t.whist[w][tid] = count;
+            count += c;
+        }
+    }
+    // exclusive scan of the 256 counts (the first four waves)
+    uint32_t incl = count;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t y = __shfl_up(incl, off, 64);
+        if (lane >= (uint32_t)off) incl += y;
+    }
+    if (tid < 256 && lane == 63) t.tmp[wave] = incl;
+    __syncthreads();
+    if (tid < 256) {
+        uint32_t before = 0;
+        for (uint32_t w = 0; w < wave; w++) before += t.tmp[w];
+        t.start[tid] = incl - count + before;
+    }
+    return count;
+}
+
+template <class KeyT>
 __global__ __launch_bounds__(SORT_THREADS) void k_onesweep(
     const KeyT* __restrict__ keys_in, const uint32_t* __restrict__ vals_in, KeyT* __restrict__ keys_out,
     uint32_t* __restrict__ vals_out, uint32_t n_max, const uint32_t* __restrict__ n_dev, uint32_t shift,
     uint32_t nbits, uint32_t flip, const uint32_t* __restrict__ bases, uint32_t* __restrict__ status,
     uint32_t* __restrict__ tile_ctr)
 {
-    __shared__ uint32_t s_tile;
-    __shared__ uint32_t s_whist[SORT_WAVES][256];
-    __shared__ uint32_t s_start[256];
+    __shared__ SortTile<KeyT> s;
     __shared__ uint32_t s_gbase[256];
-    __shared__ uint32_t s_tmp[8];
-    __shared__ KeyT s_keys[SORT_TILE];
-    __shared__ uint32_t s_vals[SORT_TILE];
-
+    __shared__ uint32_t s_tile;
     const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const uint32_t mask = (1u << nbits) - 1u;
     const uint32_t n = n_dev ? *n_dev : n_max;
     if (tid == 0) s_tile = atomicAdd(tile_ctr, 1u);
-    for (uint32_t i = tid; i < SORT_WAVES * 256; i += SORT_THREADS) (&s_whist[0][0])[i] = 0;
     __syncthreads();
     const uint32_t tile = s_tile;
     const uint32_t tile_start = tile * SORT_TILE;
     if (tile_start >= n) return;   // same for the whole block
     const uint32_t tile_n = min((uint32_t)SORT_TILE, n - tile_start);
-
     KeyT k[SORT_ITEMS];
     uint32_t v[SORT_ITEMS], rk[SORT_ITEMS], dg[SORT_ITEMS];
-    const uint64_t lanes_below = (1ull << lane) - 1ull;
-    const uint32_t wbase = wave * 64 * SORT_ITEMS;
 #pragma unroll
     for (int j = 0; j < SORT_ITEMS; j++) {
-        const uint32_t local = wbase + j * 64 + lane;
+        const uint32_t local = (wave * SORT_ITEMS + j) * 64 + lane, g = tile_start + local;
         const bool valid = local < tile_n;
-        const uint32_t g = tile_start + local;
-        KeyT key = valid ? keys_in[g] : (KeyT)0;
-        uint32_t val = valid ? (vals_in ? vals_in[g] : g) : 0u;
-        uint32_t d = digit_of(key, shift, mask, flip);
-        uint64_t peers = __ballot(valid);
-        for (uint32_t b = 0; b < nbits; b++) {
-            uint32_t bit = (d >> b) & 1u;
-            uint64_t bal = __ballot(bit);
-            peers &= bit ? bal : ~bal;
-        }
-        uint32_t pre = (uint32_t)__popcll(peers & lanes_below);
-        uint32_t cnt = (uint32_t)__popcll(peers);
-        uint32_t base = valid ? s_whist[wave][d] : 0u;
-        if (valid && pre == 0) s_whist[wave][d] = base + cnt;
-        k[j] = key;
-        v[j] = val;
-        rk[j] = base + pre;
-        dg[j] = valid ? d : 0xFFFFFFFFu;
+        k[j] = valid ? keys_in[g] : (KeyT)0;
+        v[j] = valid ? (vals_in ? vals_in[g] : g) : 0u;
     }
-    __syncthreads();
-
-    // exclusive offsets of each wave inside a digit, tile total per digit
-    const uint32_t d = tid;
-    uint32_t count = 0;
+    const uint32_t count = rank_tile(s, k, tile_n, shift, nbits, flip, rk, dg);
+    if (tid < 256) {
+        // decoupled look-back: publish this tile's count, add predecessors'
+        const uint32_t d = tid;
+        uint32_t* st = status + (size_t)tile * 256;
+        uint32_t excl = 0;
+        if (tile == 0) {
+            __hip_atomic_store(&st[d], FLAG_PREFIX | count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        } else {
+            __hip_atomic_store(&st[d], FLAG_AGG | count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            // LOOKBACK predecessors are read at once: the words come from
+            // memory past the L2, and tiles that start together look back
+            // over many
+            int t = (int)tile - 1;
+            bool open = true;
+            while (open) {
+                uint32_t w[LOOKBACK];
 #pragma unroll
-    for (int w = 0; w < SORT_WAVES; w++) {
-        uint32_t t = s_whist[w][d];
-        s_whist[w][d] = count;
-        count += t;
-    }
-    s_start[d] = block_exclusive_scan256(count, s_tmp);
-
-    // decoupled look-back: publish this tile's count, add predecessors'
-    uint32_t* st = status + (size_t)tile * 256;
-    uint32_t excl = 0;
-    if (tile == 0) {
-        __hip_atomic_store(&st[d], FLAG_PREFIX | count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    } else {
-        __hip_atomic_store(&st[d], FLAG_AGG | count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        int t = (int)tile - 1;
-        for (;;) {
-            uint32_t s = __hip_atomic_load(&status[(size_t)t * 256 + d], __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_AGENT);
-            if ((s >> 30) == 0u) {
-                __builtin_amdgcn_s_sleep(1);
-                continue;
+                for (int q = 0; q < LOOKBACK; q++)
+                    w[q] = __hip_atomic_load(&status[(size_t)(t > q ? t - q : 0) * 256 + d], __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT);
+                bool wait = false;   // not published yet: read again from there
+#pragma unroll
+                for (int q = 0; q < LOOKBACK; q++) {
+                    if (open && !wait) {
+                        if ((w[q] >> 30) == 0u) {
+                            wait = true;
+                        } else {
+                            excl += w[q] & COUNT_MASK;
+                            open = !(w[q] & FLAG_PREFIX) && t > 0;
+                            t--;
+                        }
+                    }
+                }
+                if (wait) __builtin_amdgcn_s_sleep(1);
             }
-            excl += s & COUNT_MASK;
-            if ((s & FLAG_PREFIX) || t == 0) break;
-            t--;
+            __hip_atomic_store(&st[d], FLAG_PREFIX | (excl + count), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
         }
-        __hip_atomic_store(&st[d], FLAG_PREFIX | (excl + count), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
+        s_gbase[d] = bases[d] + excl;
     }
-    s_gbase[d] = bases[d] + excl;
     __syncthreads();
-
 #pragma unroll
     for (int j = 0; j < SORT_ITEMS; j++) {
         if (dg[j] != 0xFFFFFFFFu) {
-            uint32_t pos = s_start[dg[j]] + s_whist[wave][dg[j]] + rk[j];
-            s_keys[pos] = k[j];
-            s_vals[pos] = v[j];
+            const uint32_t pos = s.start[dg[j]] + s.whist[wave][dg[j]] + rk[j];
+            s.keys[pos] = k[j];
+            s.vals[pos] = v[j];
         }
     }
     __syncthreads();
+    const uint32_t mask = (1u << nbits) - 1u;
     for (uint32_t i = tid; i < tile_n; i += SORT_THREADS) {
-        KeyT key = s_keys[i];
-        uint32_t dd = digit_of(key, shift, mask, flip);
-        uint32_t o = s_gbase[dd] + (i - s_start[dd]);
+        const KeyT key = s.keys[i];
+        const uint32_t dd = digit_of(key, shift, mask, flip);
+        const uint32_t o = s_gbase[dd] + (i - s.start[dd]);
         if (keys_out) keys_out[o] = key;
-        vals_out[o] = s_vals[i];
+        vals_out[o] = s.vals[i];
+    }
+}
+
+// All passes of a sort of at most one tile in one block: the keys stay in LDS
+// between the passes.  Replaces a fill, a histogram, a scan and a launch per
+// pass: 2003 64-bit keys over 63 bits SMALL_US.
+template <class KeyT>
+__global__ __launch_bounds__(SORT_THREADS) void k_sort_tile(const KeyT* __restrict__ keys_in,
+                                                            const uint32_t* __restrict__ vals_in,
+                                                            KeyT* __restrict__ keys_out,
+                                                            uint32_t* __restrict__ vals_out, uint32_t n_max,
+                                                            const uint32_t* __restrict__ n_dev, PassDesc pd,
+                                                            uint32_t* __restrict__ part_offsets, uint32_t part_digits)
+{
+    __shared__ SortTile<KeyT> s;
+    __shared__ uint32_t s_part[256];
+    const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const uint32_t n = n_dev ? min(*n_dev, n_max) : n_max;
+    KeyT k[SORT_ITEMS];
+    uint32_t v[SORT_ITEMS], rk[SORT_ITEMS], dg[SORT_ITEMS];
+    if (tid < 256) s_part[tid] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < SORT_ITEMS; j++) {
+        const uint32_t i = (wave * SORT_ITEMS + j) * 64 + lane;
+        const bool valid = i < n;
+        k[j] = valid ? keys_in[i] : (KeyT)0;
+        v[j] = valid ? (vals_in ? vals_in[i] : i) : 0u;
+        if (valid && part_offsets) atomicAdd(&s_part[digit_of(k[j], pd.part_shift, pd.part_mask, pd.part_flip)], 1u);
+    }
+    for (uint32_t p = 0; p < pd.passes; p++) {
+        (void)rank_tile(s, k, n, pd.shift[p], (uint32_t)__popc(pd.mask[p]), pd.flip[p], rk, dg);
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < SORT_ITEMS; j++) {
+            if (dg[j] != 0xFFFFFFFFu) {
+                const uint32_t pos = s.start[dg[j]] + s.whist[wave][dg[j]] + rk[j];
+                s.keys[pos] = k[j];
+                s.vals[pos] = v[j];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < SORT_ITEMS; j++) {
+            const uint32_t i = (wave * SORT_ITEMS + j) * 64 + lane;
+            if (i < n) {
+                k[j] = s.keys[i];
+                v[j] = s.vals[i];
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < SORT_ITEMS; j++) {
+        const uint32_t i = (wave * SORT_ITEMS + j) * 64 + lane;
+        if (i < n) {
+            if (keys_out) keys_out[i] = k[j];
+            vals_out[i] = v[j];
+        }
+    }
+    if (part_offsets) {   // exclusive scan of the partition's digit counts
+        __syncthreads();
+        if (tid < 64) {
+            uint32_t run = 0;
+            for (uint32_t b = 0; b < part_digits; b += 64) {
+                const uint32_t x = (b + lane < part_digits) ? s_part[b + lane] : 0u;
+                uint32_t incl = x;
+                for (int off = 1; off < 64; off <<= 1) {
+                    const uint32_t y = __shfl_up(incl, off, 64);
+                    if (lane >= (uint32_t)off) incl += y;
+                }
+                if (b + lane < part_digits) part_offsets[b + lane] = run + incl - x;
+                run += __shfl(incl, 63, 64);
+            }
+            if (lane == 0) part_offsets[part_digits] = n;
+        }
     }
 }
 
@@ -243,6 +385,13 @@ int32_t radix_sort_t(mrh_context* ctx, const SortArgs& a, const SortSpace* space
         pd.part_flip = a.descending ? pd.part_mask : 0u;
     }
 
+    if (tiles == 1) {
+        const auto tile = [&](auto run) {
+            return run(ctx, "sort_tile", dim3(1), dim3(SORT_THREADS), 0, k_sort_tile<KeyT>, (const KeyT*)a.keys_in,
+                       a.vals_in, (KeyT*)a.keys_out, a.vals_out, a.n_max, a.n_dev, pd, a.part_offsets, part_digits);
+        };
+        return space ? tile([](auto... x) { return launch_plain(x...); }) : tile([](auto... x) { return launch(x...); });
+    }
     const size_t meta_words = META_STATUS + (size_t)passes * tiles * 256;
     const bool plain = space != nullptr;   // a fixed workspace: no allocation, no events
     uint32_t* meta = nullptr;
@@ -276,19 +425,17 @@ int32_t radix_sort_t(mrh_context* ctx, const SortArgs& a, const SortSpace* space
     MRH_TRY(fill_u32(ctx, meta, 0u, meta_words, plain));
 
     // Each block flushes passes x 256 counters with global atomics, so the
-    // grid is sized for >= 4096 keys per block and at most 4 blocks per CU:
-    // one block per 256 keys put millions of atomics on 1024 words.
-    uint32_t hist_blocks = div_up(a.n_max, 4096u);
-    hist_blocks = std::min<uint32_t>(hist_blocks, ctx->num_cus * 4u);
+    // grid is one block a chunk and at most one a CU.
+    uint32_t hist_blocks = div_up(a.n_max, HIST_CHUNK);
+    hist_blocks = std::min<uint32_t>(hist_blocks, ctx->num_cus);
     hist_blocks = std::max<uint32_t>(hist_blocks, 1u);
-    auto run = [&](const char* name, dim3 grid, auto kernel, auto... args) -> int32_t {
-        return plain ? launch_plain(ctx, name, grid, dim3(256), 0, kernel, args...)
-                     : launch(ctx, name, grid, dim3(256), 0, kernel, args...);
+    auto run = [&](const char* name, dim3 grid, uint32_t block, auto kernel, auto... args) -> int32_t {
+        return plain ? launch_plain(ctx, name, grid, dim3(block), 0, kernel, args...)
+                     : launch(ctx, name, grid, dim3(block), 0, kernel, args...);
     };
-    static_assert(SORT_THREADS == 256, "every sort kernel runs 256-thread blocks");
-    MRH_TRY(run("sort_hist", dim3(hist_blocks), k_sort_hist<KeyT>, (const KeyT*)a.keys_in, a.n_max,
+    MRH_TRY(run("sort_hist", dim3(hist_blocks), HIST_THREADS, k_sort_hist<KeyT>, (const KeyT*)a.keys_in, a.n_max,
                 a.n_dev, pd, meta));
-    MRH_TRY(run("sort_scan", dim3(1), k_sort_scan, meta, passes, a.part_offsets, part_digits, a.n_max,
+    MRH_TRY(run("sort_scan", dim3(1), 256u, k_sort_scan, meta, passes, a.part_offsets, part_digits, a.n_max,
                 a.n_dev));
 
     const KeyT* kin = (const KeyT*)a.keys_in;
@@ -297,7 +444,7 @@ int32_t radix_sort_t(mrh_context* ctx, const SortArgs& a, const SortSpace* space
         const bool last = (p + 1 == passes);
         KeyT* kout = last ? (KeyT*)a.keys_out : (KeyT*)((p & 1) ? kb : ka);
         uint32_t* vout = last ? a.vals_out : (uint32_t*)((p & 1) ? vb : va);
-        MRH_TRY(run("sort_onesweep", dim3(tiles), k_onesweep<KeyT>, kin, vin, kout, vout, a.n_max,
+        MRH_TRY(run("sort_onesweep", dim3(tiles), (uint32_t)SORT_THREADS, k_onesweep<KeyT>, kin, vin, kout, vout, a.n_max,
                     a.n_dev, pd.shift[p], (uint32_t)__builtin_popcount(pd.mask[p]), pd.flip[p],
                     (const uint32_t*)(meta + META_HIST + p * 256),
                     meta + META_STATUS + (size_t)p * tiles * 256, meta + META_CTR + p));

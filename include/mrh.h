@@ -79,8 +79,9 @@ int32_t     mrh_profile_get(mrh_context* ctx, const char* kernel, double* total_
  *   "trace_block"         threads per block of the frame renders' traversal
  *                         kernel (128, 256, 512; two-level scenes and the
  *                         serving engine use 256)
- *   "shade_tile"          rays per tile of shade_partition 1 (512, 1024,
- *                         2048)
+ *   "shade_tile"          rays per tile of shade_partition 1 at most (512,
+ *                         1024, 2048; frames too small for four tiles a CU
+ *                         take smaller ones)
  *   "fail_alloc_after"    failure-handling tests: k > 0 makes the k-th
  *                         following device allocation of this context fail
  *                         with MRH_ERR_OOM (0 = off)

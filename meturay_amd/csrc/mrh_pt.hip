@@ -1095,7 +1095,13 @@ int32_t frame_bounce(mrh_context* ctx, const mrh_scene* s, Frame& f, float* imag
     case 6: MRH_TRY(shade_t(k_shade_tiles<false, true, true, T>, T)); break;                   \
     default: MRH_TRY(shade_t(k_shade_tiles<true, true, true, T>, T)); break;                   \
     }
-        switch (ctx->shade_tile) {
+        // Frames with fewer than four tiles a CU take smaller ones, down to 256
+        // rays: 64 tiles of 1024 rays left most of the chip idle in a 256x256
+        // preview (18.2 us a bounce, 8.2 us with 256).
+        uint32_t tile = ctx->shade_tile;
+        while (tile > 256u && f.cap < (uint64_t)tile * ctx->num_cus * 4u) tile >>= 1;
+        switch (tile) {
+        case 256: MRH_SHADE_TILES(256u); break;
         case 512: MRH_SHADE_TILES(512u); break;
         case 1024: MRH_SHADE_TILES(1024u); break;
         case 2048: MRH_SHADE_TILES(2048u); break;

@@ -553,8 +553,20 @@ __device__ inline bool vox_pixel(const VoxSetup& s, const float cube[4], uint32_
     return true;
 }
 
+constexpr uint32_t VOX_WORDS = sizeof(VoxSetup) / 4;
+union VoxWords {
+    VoxSetup s;
+    uint32_t w[VOX_WORDS];
+};
+
 // offsets == nullptr: out[t] = records of triangle t; else out[offsets[t] +
-// rank] = the records
+// rank] = the records.
+//
+// A wave takes 64 triangles: every lane sets up one (about 20 IEEE divisions),
+// then the wave rasterises them one after another, all lanes on the pixels of
+// one triangle, whose set-up is read from its lane into scalar registers.  With
+// every lane repeating each triangle's set-up a pass over 491 k triangles at
+// depth 9 took 330 us, now 197 us.
 __global__ __launch_bounds__(256) void k_voxelize(const float* __restrict__ tris, uint32_t n, float4 cube4,
                                                   uint32_t depth, const uint32_t* __restrict__ offsets,
                                                   uint32_t* __restrict__ out, uint32_t* __restrict__ prims,
@@ -566,31 +578,47 @@ __global__ __launch_bounds__(256) void k_voxelize(const float* __restrict__ tris
     const float cube[4] = {cube4.x, cube4.y, cube4.z, cube4.w};
     const uint64_t below = (1ull << lane) - 1ull;
     unsigned long long wave_total = 0ull;   // one atomic per wave, not per triangle
-    for (uint32_t t = (blockIdx.x * blockDim.x + threadIdx.x) >> 6; t < n; t += nw) {
-        VoxSetup s;
-        vox_setup(tris + 9 * (size_t)t, cube, R, s);
-        const int w = s.x1 - s.x0, h = s.y1 - s.y0;
-        const uint32_t area = (w > 0 && h > 0) ? (uint32_t)(w * h) : 0u;
-        uint32_t run = offsets ? offsets[t] : 0u;
-        for (uint32_t base = 0; base < area; base += 64u) {
-            const uint32_t k = base + lane;
-            uint32_t code = 0u;
-            bool hit = false;
-            if (k < area) hit = vox_pixel(s, cube, R, s.x0 + (int)(k % (uint32_t)w), s.y0 + (int)(k / (uint32_t)w), code);
-            const uint64_t m = __ballot(hit);
-            if (offsets && hit) {
-                const uint32_t at = run + (uint32_t)__popcll(m & below);
-                out[at] = code;
-                if (prims) prims[at] = t;
+    for (uint32_t t0 = ((blockIdx.x * blockDim.x + threadIdx.x) >> 6) * 64u; t0 < n; t0 += nw * 64u) {
+        const uint32_t cnt = min(64u, n - t0);
+        VoxWords mine = {};
+        if (lane < cnt) vox_setup(tris + 9 * (size_t)(t0 + lane), cube, R, mine.s);
+        const uint32_t run = (offsets && lane < cnt) ? offsets[t0 + lane] : 0u;
+        uint32_t records = 0;
+        for (uint32_t i = 0; i < cnt; i++) {
+            VoxWords of;
+#pragma unroll
+            for (uint32_t k = 0; k < VOX_WORDS; k++)
+                of.w[k] = (uint32_t)__builtin_amdgcn_readlane((int)mine.w[k], (int)i);
+            const VoxSetup& s = of.s;
+            const int w = s.x1 - s.x0, h = s.y1 - s.y0;
+            const uint32_t area = (w > 0 && h > 0) ? (uint32_t)(w * h) : 0u;
+            const uint32_t at0 = (uint32_t)__builtin_amdgcn_readlane((int)run, (int)i);
+            uint32_t got = 0;
+            for (uint32_t base = 0; base < area; base += 64u) {
+                const uint32_t k = base + lane;
+                uint32_t code = 0u;
+                bool hit = false;
+                if (k < area)
+                    hit = vox_pixel(s, cube, R, s.x0 + (int)(k % (uint32_t)w), s.y0 + (int)(k / (uint32_t)w), code);
+                const uint64_t m = __ballot(hit);
+                if (offsets && hit) {
+                    const uint32_t at = at0 + got + (uint32_t)__popcll(m & below);
+                    out[at] = code;
+                    if (prims) prims[at] = t0 + i;
+                }
+                got += (uint32_t)__popcll(m);
             }
-            run += (uint32_t)__popcll(m);
+            if (lane == i) records = got;
         }
-        if (!offsets && lane == 0) {
-            out[t] = run;
-            wave_total += run;
+        if (!offsets && lane < cnt) {
+            out[t0 + lane] = records;
+            wave_total += records;
         }
     }
-    if (!offsets && lane == 0 && wave_total) atomicAdd(total, wave_total);
+    if (!offsets) {
+        for (int off = 32; off > 0; off >>= 1) wave_total += __shfl_xor(wave_total, off, 64);
+        if (lane == 0 && wave_total) atomicAdd(total, wave_total);
+    }
 }
 
 // ---------------------------------------------------------------- cone trace
@@ -1461,7 +1489,7 @@ int32_t svo_voxelize_count(mrh_context* ctx, const float* d_tris, uint32_t n, co
     unsigned long long* total = (unsigned long long*)mem;
     uint32_t* counts = (uint32_t*)mem + 2;
     const float4 c4 = make_float4(cube[0], cube[1], cube[2], cube[3]);
-    const uint32_t grid = (uint32_t)std::min<uint64_t>(div_up(n, 4), (uint64_t)ctx->num_cus * 8u);
+    const uint32_t grid = (uint32_t)std::min<uint64_t>(div_up(n, 256), (uint64_t)ctx->num_cus * 8u);
     MRH_TRY(fill_u32(ctx, (uint32_t*)mem, 0u, 2));
     MRH_TRY(fill_u32(ctx, counts + n, 0u, 1));
     MRH_TRY(launch(ctx, "voxelize_count", dim3(grid), dim3(256), 0, k_voxelize, d_tris, n, c4, depth,
@@ -1480,7 +1508,7 @@ int32_t svo_voxelize_write(mrh_context* ctx, const float* d_tris, uint32_t n, co
 {
     uint32_t* counts = (uint32_t*)ctx->slot_ptr[SLOT_VOXEL] + 2;
     MRH_TRY(scan_exclusive(ctx, counts, counts, n + 1, counts + n + 1));
-    const uint32_t grid = (uint32_t)std::min<uint64_t>(div_up(n, 4), (uint64_t)ctx->num_cus * 8u);
+    const uint32_t grid = (uint32_t)std::min<uint64_t>(div_up(n, 256), (uint64_t)ctx->num_cus * 8u);
     return launch(ctx, "voxelize", dim3(grid), dim3(256), 0, k_voxelize, d_tris, n,
                   make_float4(cube[0], cube[1], cube[2], cube[3]), depth, (const uint32_t*)counts, d_codes, d_prims,
                   (unsigned long long*)nullptr);

@@ -39,22 +39,10 @@ WfpgTaps gauss_taps(float alpha)
     return taps;
 }
 
-// Utility::CocentricOctohedralWrapInt (CoordinateConversion.h:213-235):
-// fold a texel index back into [0,X) x [0,Y); an odd fold count in exactly
-// one axis mirrors both coordinates.
-__device__ inline void octa_fold(int x, int y, int X, int Y, int& ox, int& oy)
-{
-    const int sx = (x < 0) ? -2 * X - x : x;
-    const int sy = (y < 0) ? -2 * Y - y : y;
-    const int ix = sx / X, iy = sy / Y;
-    int fx = abs(sx % X), fy = abs(sy % Y);
-    if ((ix & 1) ^ (iy & 1)) {
-        fx = (X - 1) - fx;
-        fy = (Y - 1) - fy;
-    }
-    ox = fx;
-    oy = fy;
-}
+// Utility::CocentricOctohedralWrapInt (CoordinateConversion.h:213-235) for one
+// axis less than its size outside: the index is mirrored at the border it left
+// by, and the other axis (inside its own range) mirrors with it.
+__device__ inline int octa_fold(int x, int X) { return x < 0 ? -1 - x : 2 * X - 1 - x; }
 
 // Continuous index of xi in one axis of the distribution
 // (BlockPWCDistribution2D::Sample with BinarySearchInBetween): c holds the
@@ -63,31 +51,32 @@ __device__ inline void octa_fold(int x, int y, int X, int Y, int& ox, int& oy)
 // size - 1e-5.  The interval is found as the count of entries <= xi, in
 // log2(size) fixed steps: for a non-decreasing cdf (non-negative radiance)
 // that is the one interval the reference's bisection stops at.
+// The entries are c[i] * norm.
 template <int SIZE>
-__device__ inline float pwc_axis(const float* c, float xi)
+__device__ inline float pwc_axis(const float* c, float norm, float xi)
 {
     int pos = 0;
 #pragma unroll
     for (int step = SIZE / 2; step >= 1; step >>= 1)
-        pos = (c[pos + step - 1] <= xi) ? pos + step : pos;
-    if (pos == SIZE - 1 && c[SIZE - 1] <= xi) pos = SIZE;   // the steps reach at most SIZE - 1
-    if (pos == 0) return xi / c[0];
+        pos = (c[pos + step - 1] * norm <= xi) ? pos + step : pos;
+    if (pos == SIZE - 1 && c[SIZE - 1] * norm <= xi) pos = SIZE;   // the steps reach at most SIZE - 1
+    if (pos == 0) return xi / (c[0] * norm);
     if (pos == SIZE) return (float)SIZE - 1.0e-5f;
-    const float cm = c[pos - 1], cn = c[pos];
+    const float cm = c[pos - 1] * norm, cn = c[pos] * norm;
     return ((float)(pos - 1) + (xi - cm) / (cn - cm)) + 1.0f;
 }
 
 // pdf of the texel under (u,v) times 1/(4 pi) (solid angle of the map);
 // coordinates outside [0,1) (or NaN) clamp to the border texels
 template <int X, int Y, int LS>
-__device__ inline float pwc_pdf(const float* s_pdf, const float* s_py, float u, float v)
+__device__ inline float pwc_pdf(const float* s_val, const float* s_norm, const float* s_py, float u, float v)
 {
     const float fx = u * (float)X, fy = v * (float)Y;
     uint32_t ix = (fx > 0.0f) ? (uint32_t)fminf(fx, 65536.0f) : 0u;
     uint32_t iy = (fy > 0.0f) ? (uint32_t)fminf(fy, 65536.0f) : 0u;
     ix = ix >= (uint32_t)X ? X - 1 : ix;
     iy = iy >= (uint32_t)Y ? Y - 1 : iy;
-    const float p = s_pdf[iy * LS + ix] * s_py[iy];
+    const float p = (s_val[iy * LS + ix] * s_norm[iy]) * s_py[iy];
     return p * (0.25f * 0.318309886183790671538f);
 }
 
@@ -249,8 +238,9 @@ __global__ __launch_bounds__(WFPG_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
 {
     constexpr int N = X * Y;
     constexpr int LS = X + 1;            // padded row stride: lane-per-row walks hit distinct banks
-    __shared__ float s_a[Y * LS];        // field -> filtered field -> row pdfs
-    __shared__ float s_b[Y * LS];        // u-pass result -> row cdfs
+    __shared__ float s_a[Y * LS];        // field -> filtered field (a row's pdf / its s_norm)
+    __shared__ float s_b[Y * LS];        // u-pass result -> row cdfs / s_norm
+    __shared__ float s_norm[Y];          // 1 / integral of a row
     __shared__ float s_row[Y];           // marginal pdf
     __shared__ float s_cy[Y];            // marginal cdf
     __shared__ float s_cavg[PRODUCT ? PS * PS : 1], s_cmax[PRODUCT ? PS * PS : 1];   // 8x8 cells
@@ -277,10 +267,13 @@ __global__ __launch_bounds__(WFPG_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
         // this thread's first ray of the bin, loaded before the field work
         const uint32_t lo = offsets[bin], hi = offsets[bin + 1];
         uint32_t r0 = 0xFFFFFFFFu;
-        float2 x0 = make_float2(0.0f, 0.0f);
+        float2 x0 = make_float2(0.0f, 0.0f), e0 = make_float2(0.0f, 0.0f);
         if (lo + (uint32_t)tid < hi) {
             r0 = ray_ids[lo + tid];
-            if (!PRODUCT && r0 < ray_count) x0 = xi[r0];
+            if (!PRODUCT && r0 < ray_count) {
+                x0 = xi[r0];
+                if (eval_uv) e0 = eval_uv[r0];
+            }
         }
         // radiance query result: an empty texel keeps a small weight
         // (WFPGTracerKC.cuh:1316-1317)
@@ -298,7 +291,10 @@ __global__ __launch_bounds__(WFPG_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
 #pragma unroll
             for (int i = 0; i < K + 2 * WFPG_HALF; i++) {
                 int qx = x0 - WFPG_HALF + i, qy = y;
-                if (qx < 0 || qx >= X) octa_fold(qx, y, X, Y, qx, qy);
+                if (qx < 0 || qx >= X) {
+                    qx = octa_fold(qx, X);
+                    qy = Y - 1 - y;
+                }
                 w[i] = s_a[qy * LS + qx];
             }
 #pragma unroll
@@ -317,7 +313,10 @@ __global__ __launch_bounds__(WFPG_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
 #pragma unroll
             for (int i = 0; i < K + 2 * WFPG_HALF; i++) {
                 int qx = x, qy = y0 - WFPG_HALF + i;
-                if (qy < 0 || qy >= Y) octa_fold(x, qy, X, Y, qx, qy);
+                if (qy < 0 || qy >= Y) {
+                    qy = octa_fold(qy, Y);
+                    qx = X - 1 - x;
+                }
                 w[i] = s_b[qy * LS + qx];
             }
 #pragma unroll
@@ -332,30 +331,24 @@ __global__ __launch_bounds__(WFPG_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
         __syncthreads();
         if constexpr (!PRODUCT) {
             // conditional distributions, one lane of the first wave per row
-            // (GPUBlockPWCDistribution.cuh:107-156): the row total first, then
-            // the same left-to-right prefix again while the row is normalised
+            // (GPUBlockPWCDistribution.cuh:107-156): the left-to-right prefix.
+            // The rays divide by the row's integral where they look an entry
+            // up: a few of them per ray, where 64 x 64 texels were normalised
+            // by this one wave while the others waited (4,096 bins of 64 x 64,
+            // 2 M rays: 187 -> 180 us; the rays' 567 MB of scattered lines
+            // bound it).
             float m = 0.0f;                  // this lane's row total * dY
             if (tid < Y) {
-                float* ra = s_a + tid * LS;
+                const float* ra = s_a + tid * LS;
                 float* rb = s_b + tid * LS;
                 float s = 0.0f;
-    #pragma unroll 16
-                for (int x = 0; x < X; x++) s += ra[x];
-                const float sdx = s * dX;
-                const bool norm = (sdx != 0.0f);
-                const float inv = norm ? 1.0f / sdx : 1.0f;
-                float c = 0.0f;
-    #pragma unroll 16
+#pragma unroll 16
                 for (int x = 0; x < X; x++) {
-                    const float v = ra[x];
-                    c += v;
-                    if (norm) {
-                        ra[x] = v * inv;
-                        rb[x] = (c * dX) * inv;
-                    } else {
-                        rb[x] = c * dX;
-                    }
+                    s += ra[x];
+                    rb[x] = s * dX;
                 }
+                const float sdx = s * dX;
+                s_norm[tid] = (sdx != 0.0f) ? 1.0f / sdx : 1.0f;
                 m = s * dY;
             }
             // marginal over rows (:158-199) in the first wave: lane y adds the
@@ -410,15 +403,15 @@ __global__ __launch_bounds__(WFPG_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
                     u = x2.x;
                     v = x2.y;
                 } else {
-                    const float iy = pwc_axis<Y>(s_cy, x2.y);
+                    const float iy = pwc_axis<Y>(s_cy, 1.0f, x2.y);
                     int row = (int)iy;
                     row = row >= Y ? Y - 1 : (row < 0 ? 0 : row);
-                    const float ix = pwc_axis<X>(s_b + row * LS, x2.x);
+                    const float ix = pwc_axis<X>(s_b + row * LS, s_norm[row], x2.x);
                     u = ix * dX;
                     v = iy * dY;
                 }
                 out_uv[r] = make_float2(u, v);
-                out_pdf[r] = pwc_pdf<X, Y, LS>(s_a, s_row, u, v);
+                out_pdf[r] = pwc_pdf<X, Y, LS>(s_a, s_norm, s_row, u, v);
                 if (out_dir) {
                     const V3 d = octa_to_dir(u, v);   // z up; the path uses y up
                     out_dir[3 * (size_t)r] = d.y;
@@ -426,8 +419,8 @@ __global__ __launch_bounds__(WFPG_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
                     out_dir[3 * (size_t)r + 2] = d.x;
                 }
                 if (eval_uv) {
-                    const float2 e = eval_uv[r];
-                    out_eval_pdf[r] = pwc_pdf<X, Y, LS>(s_a, s_row, e.x, e.y);
+                    const float2 e = first ? e0 : eval_uv[r];
+                    out_eval_pdf[r] = pwc_pdf<X, Y, LS>(s_a, s_norm, s_row, e.x, e.y);
                 }
             }
         } else {
@@ -442,7 +435,7 @@ __global__ __launch_bounds__(WFPG_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
 template <int X, int Y>
 constexpr uint32_t wfpg_blocks_per_cu()
 {
-    const uint32_t lds = (uint32_t)(2 * Y * (X + 1) + 2 * Y) * 4u;
+    const uint32_t lds = (uint32_t)(2 * Y * (X + 1) + 3 * Y) * 4u;
     const uint32_t b = (160u * 1024u) / lds;
     return b > 8u ? 8u : b;
 }

@@ -162,7 +162,7 @@ def wfpg_render_leg(N, ctx, scene, img, torch):
               filter_alpha=1.0)
     stages = {"trace": ["trace_pt"], "shade": ["shade"], "prep": ["wfpg_prep"],
               "binning": ["bin_start", "bin_heads", "bin_own", "bin_collapse", "bin_assign", "bin_flags",
-                          "bin_runs", "wfpg_minray", "wfpg_bins", "sort_hist", "sort_scan", "sort_onesweep",
+                          "bin_runs", "wfpg_minray", "wfpg_bins", "sort_hist", "sort_scan", "sort_onesweep", "sort_tile",
                           "scan_tiles", "scan_add"],
               "field_trace": ["wfpg_trace_fields"], "field_sample": ["wfpg_fields"],
               "payload": ["payload_keys", "payload_runs", "payload_leaf_normals", "payload_node_normals",

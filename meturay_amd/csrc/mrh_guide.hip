@@ -427,8 +427,8 @@ __global__ __launch_bounds__(256) void k_svo_filter_top(uint32_t nodes, float* _
 // quarter- or half-turn quaternion stands for), rasterised conservatively at
 // the leaf resolution (edges pushed out by half a pixel along their L1
 // normal), and every covered pixel emits the leaf holding the triangle's
-// plane point under the pixel centre.  One wave per triangle: the pixels of
-// its rectangle 64 at a time, row by row, coverage by ballot; a count pass,
+// plane point under the pixel centre.  A wave walks one triangle at a time: the
+// pixels of its rectangle 64 at a time, row by row, coverage by ballot; a count pass,
 // a scan, and a write pass that places each record at its triangle's offset
 // plus its rank, so records come out triangle by triangle, row by row.
 struct VoxSetup {
@@ -624,8 +624,8 @@ __global__ __launch_bounds__(256) void k_voxelize(const float* __restrict__ tris
 // ---------------------------------------------------------------- cone trace
 // AnisoSVOctreeGPU::ConeTraceRay (AnisoSVO.cuh:767-1032) on this octree: the
 // ray in the cube's unit space, mirrored to a positive direction; a Morton
-// bit stack of the child indices taken and the parent links instead of a
-// node stack; descending into an existing child stops at a leaf, where the
+// bit stack of the child indices taken, and the ancestors' children in LDS
+// where the reference follows parent links; descending into an existing child stops at a leaf, where the
 // cone's disc (diameter^2 = 4 t^2 aperture / pi) is wider than the child's
 // voxel, or `offset` levels above the leaves; a missing child is crossed
 // past its far face.  A walk longer than CONE_MAX_STEPS steps ends as a miss.

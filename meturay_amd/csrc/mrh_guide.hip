@@ -562,11 +562,16 @@ union VoxWords {
 // offsets == nullptr: out[t] = records of triangle t; else out[offsets[t] +
 // rank] = the records.
 //
-// A wave takes 64 triangles: every lane sets up one (about 20 IEEE divisions),
-// then the wave rasterises them one after another, all lanes on the pixels of
-// one triangle, whose set-up is read from its lane into scalar registers.  With
-// every lane repeating each triangle's set-up a pass over 491 k triangles at
-// depth 9 took 330 us, now 197 us.
+// Wave w of nw takes the triangles w, w + nw, w + 2 nw, ..., up to 64 at a
+// time: every lane sets up one (about 20 IEEE divisions), then the wave
+// rasterises them one after another, all lanes on the pixels of one triangle,
+// whose set-up is read from its lane into scalar registers.  The stride spreads
+// neighbouring triangles over the waves: a room's walls, up to a million
+// pixels each, lie side by side in a mesh, and 64 neighbours in one wave are
+// walked one after another.
+// Two passes over 491 k triangles at depth 9: 428 us (713 us with every lane
+// repeating each triangle's set-up); over the 94 triangles of a room at depth
+// 10 10.5 ms (124.7 ms with 64 neighbours to a wave).
 __global__ __launch_bounds__(256) void k_voxelize(const float* __restrict__ tris, uint32_t n, float4 cube4,
                                                   uint32_t depth, const uint32_t* __restrict__ offsets,
                                                   uint32_t* __restrict__ out, uint32_t* __restrict__ prims,
@@ -578,11 +583,11 @@ __global__ __launch_bounds__(256) void k_voxelize(const float* __restrict__ tris
     const float cube[4] = {cube4.x, cube4.y, cube4.z, cube4.w};
     const uint64_t below = (1ull << lane) - 1ull;
     unsigned long long wave_total = 0ull;   // one atomic per wave, not per triangle
-    for (uint32_t t0 = ((blockIdx.x * blockDim.x + threadIdx.x) >> 6) * 64u; t0 < n; t0 += nw * 64u) {
-        const uint32_t cnt = min(64u, n - t0);
+    for (uint32_t t0 = (blockIdx.x * blockDim.x + threadIdx.x) >> 6; t0 < n; t0 += nw * 64u) {
+        const uint32_t cnt = min(64u, (n - t0 + nw - 1u) / nw), t = t0 + lane * nw;   // t: lane's, if lane < cnt
         VoxWords mine = {};
-        if (lane < cnt) vox_setup(tris + 9 * (size_t)(t0 + lane), cube, R, mine.s);
-        const uint32_t run = (offsets && lane < cnt) ? offsets[t0 + lane] : 0u;
+        if (lane < cnt) vox_setup(tris + 9 * (size_t)t, cube, R, mine.s);
+        const uint32_t run = (offsets && lane < cnt) ? offsets[t] : 0u;
         uint32_t records = 0;
         for (uint32_t i = 0; i < cnt; i++) {
             VoxWords of;
@@ -604,14 +609,14 @@ __global__ __launch_bounds__(256) void k_voxelize(const float* __restrict__ tris
                 if (offsets && hit) {
                     const uint32_t at = at0 + got + (uint32_t)__popcll(m & below);
                     out[at] = code;
-                    if (prims) prims[at] = t0 + i;
+                    if (prims) prims[at] = t0 + i * nw;
                 }
                 got += (uint32_t)__popcll(m);
             }
             if (lane == i) records = got;
         }
         if (!offsets && lane < cnt) {
-            out[t0 + lane] = records;
+            out[t] = records;
             wave_total += records;
         }
     }
@@ -1524,6 +1529,18 @@ int32_t svo_bin_rays(mrh_context* ctx, mrh_svo* s, const uint32_t* codes, uint32
 
 }  // namespace
 
+// Blocks of k_voxelize: four waves each, a wave for about 32 triangles, so that
+// few set-ups run on half-empty waves, but two to eight waves a SIMD (as far as
+// there are triangles), so that large triangles find waves of their own.  The
+// two passes over 17,280 / 94,080 / 491,520 triangles at depth 9: 96 / 151 /
+// 428 us; with 8 waves a SIMD throughout 167 / 199 / 429 us, with 16 triangles a
+// wave 96 / 174 / 430 us, with 64 and a wave a SIMD at least 96 / 180 / 447 us.
+static uint32_t vox_grid(mrh_context* ctx, uint32_t n)
+{
+    const uint64_t cus = (uint64_t)ctx->num_cus;
+    return (uint32_t)std::min<uint64_t>(div_up(n, 4), std::clamp<uint64_t>(div_up(n, 4 * 32), cus * 2u, cus * 8u));
+}
+
 // SLOT_VOXEL: a 64-bit total, counts[n + 1] (scanned in place into offsets
 // by the write half), scan scratch
 int32_t svo_voxelize_count(mrh_context* ctx, const float* d_tris, uint32_t n, const float cube[4], uint32_t depth,
@@ -1543,7 +1560,7 @@ int32_t svo_voxelize_count(mrh_context* ctx, const float* d_tris, uint32_t n, co
     unsigned long long* total = (unsigned long long*)mem;
     uint32_t* counts = (uint32_t*)mem + 2;
     const float4 c4 = make_float4(cube[0], cube[1], cube[2], cube[3]);
-    const uint32_t grid = (uint32_t)std::min<uint64_t>(div_up(n, 256), (uint64_t)ctx->num_cus * 8u);
+    const uint32_t grid = vox_grid(ctx, n);
     MRH_TRY(fill_u32(ctx, (uint32_t*)mem, 0u, 2));
     MRH_TRY(fill_u32(ctx, counts + n, 0u, 1));
     MRH_TRY(launch(ctx, "voxelize_count", dim3(grid), dim3(256), 0, k_voxelize, d_tris, n, c4, depth,
@@ -1562,7 +1579,7 @@ int32_t svo_voxelize_write(mrh_context* ctx, const float* d_tris, uint32_t n, co
 {
     uint32_t* counts = (uint32_t*)ctx->slot_ptr[SLOT_VOXEL] + 2;
     MRH_TRY(scan_exclusive(ctx, counts, counts, n + 1, counts + n + 1));
-    const uint32_t grid = (uint32_t)std::min<uint64_t>(div_up(n, 256), (uint64_t)ctx->num_cus * 8u);
+    const uint32_t grid = vox_grid(ctx, n);
     return launch(ctx, "voxelize", dim3(grid), dim3(256), 0, k_voxelize, d_tris, n,
                   make_float4(cube[0], cube[1], cube[2], cube[3]), depth, (const uint32_t*)counts, d_codes, d_prims,
                   (unsigned long long*)nullptr);

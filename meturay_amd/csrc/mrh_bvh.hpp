@@ -13,6 +13,7 @@
 #pragma once
 
 #include "mrh_internal.hpp"
+#include "mrh_walk.hpp"
 
 #include <cfloat>
 
@@ -53,22 +54,14 @@ int32_t lbvh_create(mrh_context* ctx, const float* d_tris, uint32_t n, uint32_t 
 int32_t lbvh_build_into(mrh_lbvh* b, const float* d_tris);
 void lbvh_free(mrh_lbvh* b);
 
-// Rays a wave starts with when there are few: a launch whose rays leave
-// waves free gives each wave 32 or 16 of them instead of 64, so a wave waits
-// for the longest of fewer rays (walk4_stream).  16 measured best: guided
-// 1024x768 renders 19.29 / 18.99 / 18.81 / 18.88 ms at 64 / 32 / 16 / 8.
-constexpr uint32_t TRACE_MIN_GROUP = 16;
-
-// Persistent grid of the traversal kernels: a multiple of 8 blocks (one
-// slice per XCD) of `block` threads, with room for waves of
-// TRACE_MIN_GROUP rays.
-inline uint32_t trace_grid(mrh_context* ctx, uint64_t rays, uint32_t block = 256)
+// Persistent grid of a traversal kernel.  `stream`: the kernel runs the
+// streaming walk, whose waves can take fewer than 64 rays; a one-ray-per-lane
+// kernel given blocks for such waves has its rays in the first quarter of the
+// logical blocks, on two of the eight XCDs (a 256x256 counting frame of 4 spp
+// 1.5 -> 2.2 ms).
+inline uint32_t trace_grid(mrh_context* ctx, uint64_t rays, bool stream, uint32_t block = 256)
 {
-    uint64_t want = (rays * (64 / TRACE_MIN_GROUP) + block - 1) / block;
-    uint64_t cap = (uint64_t)ctx->num_cus * ctx->trace_blocks_per_cu;
-    if (want > cap) want = cap;
-    want = (want + 7) & ~7ull;
-    return (uint32_t)(want ? want : 8);
+    return trace_blocks(rays, stream ? TRACE_MIN_GROUP : 64u, block, (uint64_t)ctx->num_cus * ctx->trace_blocks_per_cu);
 }
 
 // Overflow buffer for stack entries beyond the LDS part (per grid thread).
@@ -200,13 +193,8 @@ struct LdsStack {
     }
 };
 
-// Logical block index that gives each of the 8 XCDs (workgroups are handed
-// to XCDs round-robin) a contiguous slice of the ray range, so neighbouring
-// rays share an L2.  Requires gridDim.x % 8 == 0.
-__device__ __forceinline__ uint32_t xcd_block()
-{
-    return (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-}
+// xcd_slice of this block; requires gridDim.x % 8 == 0
+__device__ __forceinline__ uint32_t xcd_block() { return xcd_slice(blockIdx.x, gridDim.x); }
 
 // Closest (ANY = false) or any (ANY = true) hit.  Visit order: both child
 // boxes are tested at the parent; the child with the smaller entry distance

@@ -60,7 +60,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(lds_stack_wa
     const uint32_t n = counts[bounce];
     const uint32_t lb = xcd_block();
     const size_t oslot = (size_t)lb * blockDim.x + threadIdx.x;
-    if constexpr (W == 4 && L > 0 && !STATS) {
+    if constexpr (trace_streams(W, L, STATS)) {
         LdsStack<L, CAP, BS> st{s_stack, threadIdx.x, overflow, oslot};
         walk4_stream<false>(
             st, Tree4{tnodes, leaves, root, n_leaves, tmin}, lb * (BS / 64) + (threadIdx.x >> 6), gridDim.x * (BS / 64), n,
@@ -114,13 +114,14 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(lds_stack_wa
 }
 
 template <int W, int CAP, bool STATS>
-int32_t launch_trace_pt_w(mrh_context* ctx, uint32_t grid, const mrh_lbvh* b, const TreeSel& ts,
+int32_t launch_trace_pt_w(mrh_context* ctx, uint64_t rays, const mrh_lbvh* b, const TreeSel& ts,
                           const PathBuf& in, uint32_t* counts, uint32_t bounce, float tmin, float tmax,
                           const HitBuf& hit)
 {
     const uint32_t root = ts.root;
     const uint32_t lds = ctx->trace_lds_entries;
     const uint32_t bs = ctx->trace_block;
+    const uint32_t grid = trace_grid(ctx, rays, trace_streams(W, lds, STATS), bs);
     uint2* ovf = nullptr;
     MRH_TRY(trace_overflow(ctx, grid, CAP, lds, &ovf, bs));
     const char* name = STATS ? "trace_pt_stats" : "trace_pt";
@@ -149,17 +150,17 @@ int32_t launch_trace_pt_w(mrh_context* ctx, uint32_t grid, const mrh_lbvh* b, co
 }
 
 template <bool STATS>
-int32_t launch_trace_pt(mrh_context* ctx, uint32_t grid, const mrh_lbvh* b, const PathBuf& in, uint32_t* counts,
+int32_t launch_trace_pt(mrh_context* ctx, uint64_t rays, const mrh_lbvh* b, const PathBuf& in, uint32_t* counts,
                         uint32_t bounce, float tmin, float tmax, const HitBuf& hit)
 {
     TreeSel ts;
     MRH_TRY(select_tree(ctx, b, ts));
     if (ts.width == 4) {
-        if (ts.cap == 64) return launch_trace_pt_w<4, 64, STATS>(ctx, grid, b, ts, in, counts, bounce, tmin, tmax, hit);
-        return launch_trace_pt_w<4, 128, STATS>(ctx, grid, b, ts, in, counts, bounce, tmin, tmax, hit);
+        if (ts.cap == 64) return launch_trace_pt_w<4, 64, STATS>(ctx, rays, b, ts, in, counts, bounce, tmin, tmax, hit);
+        return launch_trace_pt_w<4, 128, STATS>(ctx, rays, b, ts, in, counts, bounce, tmin, tmax, hit);
     }
-    if (ts.cap == 64) return launch_trace_pt_w<2, 64, STATS>(ctx, grid, b, ts, in, counts, bounce, tmin, tmax, hit);
-    return launch_trace_pt_w<2, 128, STATS>(ctx, grid, b, ts, in, counts, bounce, tmin, tmax, hit);
+    if (ts.cap == 64) return launch_trace_pt_w<2, 64, STATS>(ctx, rays, b, ts, in, counts, bounce, tmin, tmax, hit);
+    return launch_trace_pt_w<2, 128, STATS>(ctx, rays, b, ts, in, counts, bounce, tmin, tmax, hit);
 }
 
 // Two-level scenes: the top tree over the instances, then the hit mesh's
@@ -182,7 +183,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(lds_stack_w
     const uint32_t n = counts[bounce];
     const uint32_t lb = xcd_block();
     const size_t oslot = (size_t)lb * blockDim.x + threadIdx.x;
-    if constexpr (W == 4 && L > 0 && !STATS) {
+    if constexpr (trace_streams(W, L, STATS)) {
         LdsStack<L, CAP, 256> st{s_stack, threadIdx.x, overflow, oslot};
         walk2l_stream(
             st, top4, top_leaves, top_root, n_inst, inst, mesh_nodes, leaves, tmin, lb * 4 + (threadIdx.x >> 6),
@@ -255,11 +256,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(lds_stack_w
 }
 
 template <int W, int CAP, bool STATS>
-int32_t launch_trace_pt2_w(mrh_context* ctx, uint32_t grid, const mrh_scene* s, const PathBuf& in,
+int32_t launch_trace_pt2_w(mrh_context* ctx, uint64_t rays, const mrh_scene* s, const PathBuf& in,
                            uint32_t* counts, uint32_t bounce, float tmin, float tmax, const HitBuf& hit)
 {
     const mrh_lbvh* top = s->bvh;
     const uint32_t lds = ctx->trace_lds_entries;
+    const uint32_t grid = trace_grid(ctx, rays, trace_streams(W, lds, STATS));
     uint2* ovf = nullptr;
     MRH_TRY(trace_overflow(ctx, grid, CAP, lds, &ovf));
     const char* name = STATS ? "trace_pt_stats" : "trace_pt";
@@ -282,7 +284,7 @@ int32_t launch_trace_pt2_w(mrh_context* ctx, uint32_t grid, const mrh_scene* s, 
 }
 
 template <bool STATS>
-int32_t launch_trace_pt2(mrh_context* ctx, uint32_t grid, const mrh_scene* s, const PathBuf& in, uint32_t* counts,
+int32_t launch_trace_pt2(mrh_context* ctx, uint64_t rays, const mrh_scene* s, const PathBuf& in, uint32_t* counts,
                          uint32_t bounce, float tmin, float tmax, const HitBuf& hit)
 {
     const uint32_t w = (ctx->trace_width == 4) ? 4u : 2u;
@@ -290,11 +292,11 @@ int32_t launch_trace_pt2(mrh_context* ctx, uint32_t grid, const mrh_scene* s, co
     if (need > 128)
         return fail(ctx, MRH_ERR_UNSUPPORTED, "two-level trees need %u stack entries (at most 128)", need);
     if (w == 4) {
-        if (need <= 64) return launch_trace_pt2_w<4, 64, STATS>(ctx, grid, s, in, counts, bounce, tmin, tmax, hit);
-        return launch_trace_pt2_w<4, 128, STATS>(ctx, grid, s, in, counts, bounce, tmin, tmax, hit);
+        if (need <= 64) return launch_trace_pt2_w<4, 64, STATS>(ctx, rays, s, in, counts, bounce, tmin, tmax, hit);
+        return launch_trace_pt2_w<4, 128, STATS>(ctx, rays, s, in, counts, bounce, tmin, tmax, hit);
     }
-    if (need <= 64) return launch_trace_pt2_w<2, 64, STATS>(ctx, grid, s, in, counts, bounce, tmin, tmax, hit);
-    return launch_trace_pt2_w<2, 128, STATS>(ctx, grid, s, in, counts, bounce, tmin, tmax, hit);
+    if (need <= 64) return launch_trace_pt2_w<2, 64, STATS>(ctx, rays, s, in, counts, bounce, tmin, tmax, hit);
+    return launch_trace_pt2_w<2, 128, STATS>(ctx, rays, s, in, counts, bounce, tmin, tmax, hit);
 }
 
 // One launch over all partitions of a bounce (see shade_ray); with NEE a
@@ -1032,16 +1034,15 @@ int32_t frame_bounce(mrh_context* ctx, const mrh_scene* s, Frame& f, float* imag
     const float tmin = (bounce == 0) ? f.cam.near_d : 0.0f;
     const float tmax = (bounce == 0) ? f.cam.far_d : FLT_MAX;
     const uint32_t grid = stride_grid(ctx, f.cap, 256);
-    const uint32_t tgrid = trace_grid(ctx, f.cap, s->two_level ? 256u : ctx->trace_block);
     const float4* lv = s->two_level ? (const float4*)s->leaves : (const float4*)b->leaves;
     HitBuf hb = f.hit;
     if (s->two_level) {
-        if (f.count_traversal) MRH_TRY(launch_trace_pt2<true>(ctx, tgrid, s, in, f.counts, bounce, tmin, tmax, hb));
-        else MRH_TRY(launch_trace_pt2<false>(ctx, tgrid, s, in, f.counts, bounce, tmin, tmax, hb));
+        if (f.count_traversal) MRH_TRY(launch_trace_pt2<true>(ctx, f.cap, s, in, f.counts, bounce, tmin, tmax, hb));
+        else MRH_TRY(launch_trace_pt2<false>(ctx, f.cap, s, in, f.counts, bounce, tmin, tmax, hb));
     } else {
         hb.inst = nullptr;
-        if (f.count_traversal) MRH_TRY(launch_trace_pt<true>(ctx, tgrid, b, in, f.counts, bounce, tmin, tmax, hb));
-        else MRH_TRY(launch_trace_pt<false>(ctx, tgrid, b, in, f.counts, bounce, tmin, tmax, hb));
+        if (f.count_traversal) MRH_TRY(launch_trace_pt<true>(ctx, f.cap, b, in, f.counts, bounce, tmin, tmax, hb));
+        else MRH_TRY(launch_trace_pt<false>(ctx, f.cap, b, in, f.counts, bounce, tmin, tmax, hb));
     }
     const bool tiles = ctx->shade_partition == 1;
     if (!tiles) {

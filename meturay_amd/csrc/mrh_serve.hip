@@ -117,7 +117,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(lds_stack_w
     const uint32_t n = hdr->n_total;
     const uint32_t lb = xcd_block();
     const size_t oslot = (size_t)lb * blockDim.x + threadIdx.x;
-    if constexpr (W == 4 && L > 0) {
+    if constexpr (trace_streams(W, L, false)) {
         LdsStack<L, CAP, 256> st{s_stack, threadIdx.x, overflow, oslot};
         walk4_stream<false>(
             st, Tree4{nullptr, nullptr, 0u, 0u, 0.0f}, lb * 4 + (threadIdx.x >> 6), gridDim.x * 4, n,
@@ -724,10 +724,11 @@ int32_t step_launches(mrh_server* s, uint32_t par, uint32_t v)
     MRH_TRY(fill_u32(ctx, s->d_res, 0u, RES_WORDS));
     MRH_TRY(launch(ctx, "serve_raygen", dim3(stride_grid(ctx, s->cap, 256)), dim3(256), 0, k_serve_raygen,
                    (const StepHdr*)s->d_hdr, (const SlotDev*)s->d_slots, in, s->slot_of[par]));
-    const uint32_t tgrid = trace_grid(ctx, s->buf_cap);
     const uint32_t lds = ctx->trace_lds_entries;
     uint32_t w, cap;
     tree_shape(s, w, cap);
+    const uint32_t tgrid = trace_grid(ctx, s->buf_cap, trace_streams(w, lds, false));
+    const uint32_t tgrid2 = trace_grid(ctx, s->buf_cap, false);   // k_serve_trace2; no larger
     uint2* ovf = nullptr;
     MRH_TRY(trace_overflow(ctx, tgrid, (v & 4u) ? 128u : cap, lds, &ovf));
 #define MRH_SERVE_TRACE(W, C, LV)                                                                             \
@@ -755,7 +756,7 @@ int32_t step_launches(mrh_server* s, uint32_t par, uint32_t v)
 #undef MRH_SERVE_TRACE
     if (v & 4u) {
 #define MRH_SERVE_TRACE2(W, LV)                                                                                 \
-    MRH_TRY(launch(ctx, "serve_trace", dim3(tgrid), dim3(256), 0, k_serve_trace2<W, LV>, (const StepHdr*)s->d_hdr, \
+    MRH_TRY(launch(ctx, "serve_trace", dim3(tgrid2), dim3(256), 0, k_serve_trace2<W, LV>, (const StepHdr*)s->d_hdr, \
                    (const SlotDev*)s->d_slots, in, in_slot, s->hit, ovf))
 #define MRH_SERVE_TRACE2_L(W)                                                    \
     switch (lds) {                                                               \

@@ -20,7 +20,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(lds_stack_w
     __shared__ u32x2 s_stack[L > 0 ? L * 256 : 1];
     const uint32_t lb = xcd_block();
     const size_t oslot = (size_t)lb * blockDim.x + threadIdx.x;
-    if constexpr (W == 4 && L > 0 && !STATS) {
+    if constexpr (trace_streams(W, L, STATS)) {
         LdsStack<L, CAP, 256> st{s_stack, threadIdx.x, overflow, oslot};
         walk4_stream<ANY>(
             st, Tree4{tnodes, leaves, root, n_leaves, tmin}, lb * 4 + (threadIdx.x >> 6), gridDim.x * 4, n,
@@ -76,9 +76,9 @@ template <int W, bool ANY, bool STATS, int CAP>
 int32_t trace_cap(mrh_context* ctx, const mrh_lbvh* b, const TreeSel& ts, const float* rays, uint32_t n,
                   uint32_t pitch, float tmin, uint32_t* prim, float* t, float* bary, uint32_t* stats)
 {
-    const uint32_t grid = trace_grid(ctx, n);
     const char* name = ANY ? "trace_any" : (STATS ? "trace_closest_stats" : "trace_closest");
     const uint32_t lds = ctx->trace_lds_entries;
+    const uint32_t grid = trace_grid(ctx, n, trace_streams(W, lds, STATS));
     uint2* ovf = nullptr;
     MRH_TRY(trace_overflow(ctx, grid, CAP, lds, &ovf));
 #define MRH_TRACE_L(LV)                                                                                     \

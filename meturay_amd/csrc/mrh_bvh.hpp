@@ -118,8 +118,8 @@ struct TraceResult {
 // PrivateStack keeps the whole stack in a private array (scratch memory,
 // which the L2 writes back to HBM).  LdsStack keeps the first L entries of
 // every thread in LDS, entry-major and thread-minor so a wave's accesses
-// spread over the banks, and spills deeper entries to the thread's own slice
-// of a global overflow buffer.
+// spread over the banks, and spills deeper entries to a global overflow buffer
+// (spill_base).
 template <int N>
 struct PrivateStack {
     static constexpr int CAP = N;
@@ -161,9 +161,9 @@ struct LdsStack {
     static constexpr int LDS_ENTRIES = L;
     lds_u32x2* s;         // [L][BLOCK] (code, entry distance)
     uint32_t slot;        // threadIdx.x
-    uint2* overflow;      // this thread's slice, [N - L]
+    uint2* overflow;      // this thread's entries, SPILL_STRIDE apart
     __device__ __forceinline__ LdsStack(u32x2* entries, uint32_t sl, uint2* ovf, size_t oslot)
-        : s((lds_u32x2*)entries), slot(sl), overflow(ovf + oslot * (size_t)(N > L ? N - L : 0))
+        : s((lds_u32x2*)entries), slot(sl), overflow(ovf + spill_base(oslot, N > L ? N - L : 0))
     {
     }
     __device__ __forceinline__ void put(int i, uint32_t n, float d)
@@ -171,7 +171,7 @@ struct LdsStack {
         if (i < L) {
             put_lds(i, n, d);
         } else {
-            overflow[i - L] = make_uint2(n, __float_as_uint(d));
+            overflow[(i - L) * (int)SPILL_STRIDE] = make_uint2(n, __float_as_uint(d));
         }
     }
     // entry i < L, no check
@@ -186,7 +186,7 @@ struct LdsStack {
             n = e.x;
             d = __uint_as_float(e.y);
         } else {
-            const uint2 e = overflow[i - L];
+            const uint2 e = overflow[(i - L) * (int)SPILL_STRIDE];
             n = e.x;
             d = __uint_as_float(e.y);
         }

@@ -16,6 +16,7 @@ SRC = r"""
 #include "mrh_walk.hpp"
 extern "C" uint32_t blocks(uint64_t n, uint32_t group, uint32_t block, uint64_t most) { return mrh::trace_blocks(n, group, block, most); }
 extern "C" int streams(uint32_t w, uint32_t lds, int counting) { return mrh::trace_streams(w, lds, counting != 0); }
+extern "C" uint64_t spill(uint64_t t, uint32_t entries, uint32_t e) { return mrh::spill_base(t, entries) + e * mrh::SPILL_STRIDE; }
 extern "C" uint32_t slice(uint32_t b, uint32_t n) { return mrh::xcd_slice(b, n); }
 """
 
@@ -29,6 +30,7 @@ def rules(tmp_path_factory):
                     os.path.join(ROOT, "meturay_amd", "csrc"), str(d / "w.cpp"), "-o", so], check=True)
     lib = C.CDLL(so)
     lib.blocks.argtypes = [C.c_uint64, C.c_uint32, C.c_uint32, C.c_uint64]
+    lib.spill.argtypes, lib.spill.restype = [C.c_uint64, C.c_uint32, C.c_uint32], C.c_uint64
     return lib
 
 
@@ -56,3 +58,15 @@ def test_one_ray_kernels_fill_every_xcd(rules, block, most):
                                                         (2, 8, 0, 0), (2, 0, 1, 0)])
 def test_only_the_streaming_walk_takes_small_groups(rules, width, lds, counting, streams):
     assert rules.streams(width, lds, counting) == streams
+
+
+@pytest.mark.parametrize("entries", [1, 8, 56, 120])
+def test_spilled_entries_of_a_wave_share_lines(rules, entries):
+    """8-byte entries: a depth of 64 lanes is 512 consecutive bytes, and no two
+    (thread, depth) share a place in threads * entries of them."""
+    threads = 3 * 64
+    at = [[rules.spill(t, entries, e) for t in range(threads)] for e in range(entries)]
+    assert sorted(sum(at, [])) == list(range(threads * entries))
+    for row in at:
+        for w in range(0, threads, 64):
+            assert row[w:w + 64] == list(range(row[w], row[w] + 64))

@@ -54,14 +54,10 @@ int32_t lbvh_create(mrh_context* ctx, const float* d_tris, uint32_t n, uint32_t 
 int32_t lbvh_build_into(mrh_lbvh* b, const float* d_tris);
 void lbvh_free(mrh_lbvh* b);
 
-// Persistent grid of a traversal kernel.  `stream`: the kernel runs the
-// streaming walk, whose waves can take fewer than 64 rays; a one-ray-per-lane
-// kernel given blocks for such waves has its rays in the first quarter of the
-// logical blocks, on two of the eight XCDs (a 256x256 counting frame of 4 spp
-// 1.5 -> 2.2 ms).
+// Persistent grid of a traversal kernel
 inline uint32_t trace_grid(mrh_context* ctx, uint64_t rays, bool stream, uint32_t block = 256)
 {
-    return trace_blocks(rays, stream ? TRACE_MIN_GROUP : 64u, block, (uint64_t)ctx->num_cus * ctx->trace_blocks_per_cu);
+    return trace_blocks(rays, stream, block, (uint64_t)ctx->num_cus * ctx->trace_blocks_per_cu);
 }
 
 // Overflow buffer for stack entries beyond the LDS part (per grid thread).
@@ -192,6 +188,24 @@ struct LdsStack {
         }
     }
 };
+
+// A block's share of a streaming walk of n rays: `waves` waves take `group`
+// rays at a time, this one is number `wave` of them; lb is the logical block.
+struct WalkShare {
+    uint32_t lb, wave, waves, group;
+};
+// false: no share; requires gridDim.x % 8 == 0
+template <int BLOCK>
+__device__ __forceinline__ bool walk_share(uint32_t n, WalkShare& w)
+{
+    const WalkSplit s = walk_split(n, gridDim.x, BLOCK / 64);
+    if (blockIdx.x >= s.used) return false;
+    w.lb = xcd_slice(blockIdx.x, s.used);
+    w.wave = w.lb * (BLOCK / 64) + (threadIdx.x >> 6);
+    w.waves = s.used * (BLOCK / 64);
+    w.group = s.group;
+    return true;
+}
 
 // xcd_slice of this block; requires gridDim.x % 8 == 0
 __device__ __forceinline__ uint32_t xcd_block() { return xcd_slice(blockIdx.x, gridDim.x); }
@@ -619,8 +633,8 @@ __device__ __forceinline__ uint32_t rank_below(uint64_t mask)
 constexpr uint32_t WALK_REFILL = 48;
 
 // Closest / any hits of rays [0, n) over the 4-wide tree, for a wave of a
-// persistent grid of `waves`: rays group, group + stride, ... in groups of G
-// (64; 32 or 16 when there are fewer rays than lanes).  fetch(i, o, d, tmax)
+// persistent grid: rays group, group + stride, ... in groups of G (walk_split;
+// below 64 only where one stride covers all rays).  fetch(i, o, d, tmax)
 // reads ray i, emit(i, leaf, t, ba, bb) takes its result.
 //
 // Every ray is walked in traverse4's order, with two changes in how the
@@ -655,13 +669,11 @@ struct Tree4 {
 };
 
 template <bool ANY, class Stack, class Fetch, class Emit>
-__device__ __forceinline__ void walk4_stream(Stack& st, Tree4 tr, uint32_t wave, uint32_t waves, uint32_t n,
-                                             Fetch&& fetch, Emit&& emit)
+__device__ __forceinline__ void walk4_stream(Stack& st, Tree4 tr, const WalkShare& share, uint32_t n, Fetch&& fetch,
+                                             Emit&& emit)
 {
-    uint32_t G = 64u;
-    while (G > TRACE_MIN_GROUP && (uint64_t)waves * (G >> 1) >= n) G >>= 1;
-    const uint32_t stride = waves * G;
-    uint32_t group = __builtin_amdgcn_readfirstlane(wave) * G, used = 0;   // next rays of the wave
+    const uint32_t G = share.group, stride = share.waves * G;
+    uint32_t group = __builtin_amdgcn_readfirstlane(share.wave) * G, used = 0;   // next rays of the wave
     uint32_t ray = NO_HIT;
     Walk4 w;
     w.begin(v3(0.0f, 0.0f, 0.0f), v3(0.0f, 0.0f, 0.0f), 0.0f, NO_HIT);
@@ -919,13 +931,11 @@ __device__ __forceinline__ void walk2l_stream(Stack& st, const float4* __restric
                                               const float4* __restrict__ top_leaves, uint32_t top_root,
                                               uint32_t n_inst, const float4* __restrict__ inst,
                                               const float4* __restrict__ mesh_nodes,
-                                              const float4* __restrict__ leaves, float tmin, uint32_t wave,
-                                              uint32_t waves, uint32_t n, Fetch&& fetch, Emit&& emit)
+                                              const float4* __restrict__ leaves, float tmin,
+                                              const WalkShare& share, uint32_t n, Fetch&& fetch, Emit&& emit)
 {
-    uint32_t G = 64u;
-    while (G > TRACE_MIN_GROUP && (uint64_t)waves * (G >> 1) >= n) G >>= 1;
-    const uint32_t stride = waves * G;
-    uint32_t group = __builtin_amdgcn_readfirstlane(wave) * G, used = 0;
+    const uint32_t G = share.group, stride = share.waves * G;
+    uint32_t group = __builtin_amdgcn_readfirstlane(share.wave) * G, used = 0;
     uint32_t ray = NO_HIT;
     Walk2L s;
     s.begin(v3(0.0f, 0.0f, 0.0f), v3(0.0f, 0.0f, 0.0f), 0.0f, top4, NO_HIT, n_inst);

@@ -58,12 +58,12 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(lds_stack_wa
 {
     __shared__ u32x2 s_stack[L > 0 ? L * BS : 1];
     const uint32_t n = counts[bounce];
-    const uint32_t lb = xcd_block();
-    const size_t oslot = (size_t)lb * blockDim.x + threadIdx.x;
     if constexpr (trace_streams(W, L, STATS)) {
-        LdsStack<L, CAP, BS> st{s_stack, threadIdx.x, overflow, oslot};
+        WalkShare share;
+        if (!walk_share<BS>(n, share)) return;
+        LdsStack<L, CAP, BS> st{s_stack, threadIdx.x, overflow, (size_t)share.lb * BS + threadIdx.x};
         walk4_stream<false>(
-            st, Tree4{tnodes, leaves, root, n_leaves, tmin}, lb * (BS / 64) + (threadIdx.x >> 6), gridDim.x * (BS / 64), n,
+            st, Tree4{tnodes, leaves, root, n_leaves, tmin}, share, n,
             [&](uint32_t i, V3& o, V3& d, float& tm, Tree4&) {
                 o = v3(in.ox[i], in.oy[i], in.oz[i]);
                 d = v3(in.dx[i], in.dy[i], in.dz[i]);
@@ -79,6 +79,8 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(lds_stack_wa
             });
         return;
     }
+    const uint32_t lb = xcd_block();
+    const size_t oslot = (size_t)lb * blockDim.x + threadIdx.x;
     uint64_t visits = 0, tests = 0;
     for (uint32_t i = lb * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const V3 o = v3(in.ox[i], in.oy[i], in.oz[i]);
@@ -181,13 +183,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(lds_stack_w
 {
     __shared__ u32x2 s_stack[L > 0 ? L * 256 : 1];
     const uint32_t n = counts[bounce];
-    const uint32_t lb = xcd_block();
-    const size_t oslot = (size_t)lb * blockDim.x + threadIdx.x;
     if constexpr (trace_streams(W, L, STATS)) {
-        LdsStack<L, CAP, 256> st{s_stack, threadIdx.x, overflow, oslot};
+        WalkShare share;
+        if (!walk_share<256>(n, share)) return;
+        LdsStack<L, CAP, 256> st{s_stack, threadIdx.x, overflow, (size_t)share.lb * 256 + threadIdx.x};
         walk2l_stream(
-            st, top4, top_leaves, top_root, n_inst, inst, mesh_nodes, leaves, tmin, lb * 4 + (threadIdx.x >> 6),
-            gridDim.x * 4, n,
+            st, top4, top_leaves, top_root, n_inst, inst, mesh_nodes, leaves, tmin, share, n,
             [&](uint32_t i, V3& o, V3& d, float& tm) {
                 o = v3(in.ox[i], in.oy[i], in.oz[i]);
                 d = v3(in.dx[i], in.dy[i], in.dz[i]);
@@ -208,6 +209,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(lds_stack_w
             });
         return;
     }
+    const uint32_t lb = xcd_block();
+    const size_t oslot = (size_t)lb * blockDim.x + threadIdx.x;
     uint64_t visits = 0, tests = 0;
     for (uint32_t i = lb * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const V3 o = v3(in.ox[i], in.oy[i], in.oz[i]);

@@ -115,12 +115,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(lds_stack_w
 {
     __shared__ u32x2 s_stack[L > 0 ? L * 256 : 1];
     const uint32_t n = hdr->n_total;
-    const uint32_t lb = xcd_block();
-    const size_t oslot = (size_t)lb * blockDim.x + threadIdx.x;
     if constexpr (trace_streams(W, L, false)) {
-        LdsStack<L, CAP, 256> st{s_stack, threadIdx.x, overflow, oslot};
+        WalkShare share;
+        if (!walk_share<256>(n, share)) return;
+        LdsStack<L, CAP, 256> st{s_stack, threadIdx.x, overflow, (size_t)share.lb * 256 + threadIdx.x};
         walk4_stream<false>(
-            st, Tree4{nullptr, nullptr, 0u, 0u, 0.0f}, lb * 4 + (threadIdx.x >> 6), gridDim.x * 4, n,
+            st, Tree4{nullptr, nullptr, 0u, 0u, 0.0f}, share, n,
             [&](uint32_t i, V3& o, V3& d, float& tmax, Tree4& tr) {
                 const SlotDev& sd = slots[in_slot[i]];
                 if (sd.two) return false;   // traced by k_serve_trace2
@@ -143,6 +143,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(lds_stack_w
             });
         return;
     }
+    const uint32_t lb = xcd_block();
+    const size_t oslot = (size_t)lb * blockDim.x + threadIdx.x;
     for (uint32_t i = lb * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const SlotDev& sd = slots[in_slot[i]];
         if (sd.two) continue;   // traced by k_serve_trace2

@@ -18,12 +18,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(lds_stack_w
                                                uint2* __restrict__ overflow)
 {
     __shared__ u32x2 s_stack[L > 0 ? L * 256 : 1];
-    const uint32_t lb = xcd_block();
-    const size_t oslot = (size_t)lb * blockDim.x + threadIdx.x;
     if constexpr (trace_streams(W, L, STATS)) {
-        LdsStack<L, CAP, 256> st{s_stack, threadIdx.x, overflow, oslot};
+        WalkShare share;
+        if (!walk_share<256>(n, share)) return;
+        LdsStack<L, CAP, 256> st{s_stack, threadIdx.x, overflow, (size_t)share.lb * 256 + threadIdx.x};
         walk4_stream<ANY>(
-            st, Tree4{tnodes, leaves, root, n_leaves, tmin}, lb * 4 + (threadIdx.x >> 6), gridDim.x * 4, n,
+            st, Tree4{tnodes, leaves, root, n_leaves, tmin}, share, n,
             [&](uint32_t i, V3& o, V3& d, float& tmax, Tree4&) {
                 o = v3(rays[i], rays[(size_t)pitch + i], rays[2 * (size_t)pitch + i]);
                 d = v3(rays[3 * (size_t)pitch + i], rays[4 * (size_t)pitch + i], rays[5 * (size_t)pitch + i]);
@@ -43,6 +43,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(lds_stack_w
             });
         return;
     }
+    const uint32_t lb = xcd_block();
+    const size_t oslot = (size_t)lb * blockDim.x + threadIdx.x;
     for (uint32_t i = lb * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const V3 o = v3(rays[i], rays[(size_t)pitch + i], rays[2 * (size_t)pitch + i]);
         const V3 d = v3(rays[3 * (size_t)pitch + i], rays[4 * (size_t)pitch + i], rays[5 * (size_t)pitch + i]);

@@ -7,25 +7,56 @@
 
 namespace mrh {
 
-// Rays a wave starts with when there are few: a launch whose rays leave
-// waves free gives each wave 32 or 16 of them instead of 64, so a wave waits
-// for the longest of fewer rays (walk4_stream).  16 measured best: guided
-// 1024x768 renders 19.29 / 18.99 / 18.81 / 18.88 ms at 64 / 32 / 16 / 8.
+// Few rays: a wave of the streaming walk starts with 32 or 16 instead of 64, so
+// that it waits for the longest of fewer rays, as long as that makes no more
+// than TRACE_SPLIT_WAVES waves, two a SIMD.  Past that the chip is busy, and
+// waves of fewer rays only issue more.  Closest hits, 20,000 triangles: 50,000 /
+// 100,000 / 140,000 / 200,000 rays in 100 / 105 / 118 / 142 us; split up to four
+// waves a SIMD 111 / 116 / 118 / 142, up to eight 113 / 156 / 152 / 192.  500,000
+// triangles and 50,000 rays: 232 us; up to one wave a SIMD 248.
 constexpr uint32_t TRACE_MIN_GROUP = 16;
+constexpr uint32_t TRACE_SPLIT_WAVES = 2048;
 
 // Whether a traversal kernel runs the streaming walk, whose waves can take
 // fewer than 64 rays; the others walk one ray a lane (the binary tree, the
 // counting walk, a stack without an LDS part).
 constexpr bool trace_streams(uint32_t width, uint32_t lds, bool counting) { return width == 4 && lds > 0 && !counting; }
 
-// Blocks of `block` threads for `rays` rays, `group` of them to a wave: a
-// multiple of 8 (one slice per XCD), at most `most` rounded up to one.
-constexpr uint32_t trace_blocks(uint64_t rays, uint32_t group, uint32_t block, uint64_t most)
+// Waves for `rays` rays, `group` to a wave
+constexpr uint64_t trace_waves(uint64_t rays, uint32_t group) { return (rays + group - 1) / group; }
+
+// Blocks of `block` threads for up to `rays` rays: a multiple of 8 (one slice
+// per XCD), at most `most` rounded up to one.  A streaming walk of few rays
+// gets the waves that walk_split spreads them over.
+constexpr uint32_t trace_blocks(uint64_t rays, bool stream, uint32_t block, uint64_t most)
 {
-    const uint64_t lanes = rays * (64 / group);
-    const uint64_t want = (lanes + block - 1) / block;
+    uint64_t waves = trace_waves(rays, 64);
+    if (stream) {
+        const uint64_t small = trace_waves(rays, TRACE_MIN_GROUP);
+        const uint64_t split = small < TRACE_SPLIT_WAVES ? small : TRACE_SPLIT_WAVES;
+        waves = waves > split ? waves : split;
+    }
+    const uint64_t want = (waves * 64 + block - 1) / block;
     const uint64_t some = want < most ? want : most;
     return (uint32_t)(some ? (some + 7) & ~7ull : 8);
+}
+
+// How a streaming walk of n rays uses a grid of `blocks` blocks (a multiple of
+// 8) of `waves` waves: `group` rays to a wave to start with, in the first
+// `used` blocks, a multiple of 8, so that every XCD has its share: 300,000 rays
+// on 4,688 of 8,192 waves counted from the first logical block lie on five XCDs
+// of eight (255 us in 20,000 triangles, 178 us so).
+struct WalkSplit {
+    uint32_t group, used;
+};
+constexpr WalkSplit walk_split(uint32_t n, uint32_t blocks, uint32_t waves)
+{
+    const uint64_t all = (uint64_t)blocks * waves, split = all < TRACE_SPLIT_WAVES ? all : TRACE_SPLIT_WAVES;
+    uint32_t group = 64;
+    while (group > TRACE_MIN_GROUP && trace_waves(n, group / 2) <= split) group /= 2;
+    const uint64_t need = (trace_waves(n, group) + waves - 1) / waves;
+    const uint64_t used = need ? (need + 7) & ~7ull : 8;
+    return {group, used < blocks ? (uint32_t)used : blocks};
 }
 
 // Logical index of block `b` of `blocks` (a multiple of 8) that gives each of

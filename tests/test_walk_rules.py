@@ -14,7 +14,13 @@ MOST = 256 * 8   # blocks of the whole chip at eight a CU
 
 SRC = r"""
 #include "mrh_walk.hpp"
-extern "C" uint32_t blocks(uint64_t n, uint32_t group, uint32_t block, uint64_t most) { return mrh::trace_blocks(n, group, block, most); }
+extern "C" uint32_t blocks(uint64_t n, int stream, uint32_t block, uint64_t most) { return mrh::trace_blocks(n, stream != 0, block, most); }
+extern "C" void split(uint32_t n, uint32_t blocks, uint32_t waves, uint32_t* out)
+{
+    const mrh::WalkSplit s = mrh::walk_split(n, blocks, waves);
+    out[0] = s.group;
+    out[1] = s.used;
+}
 extern "C" int streams(uint32_t w, uint32_t lds, int counting) { return mrh::trace_streams(w, lds, counting != 0); }
 extern "C" uint64_t spill(uint64_t t, uint32_t entries, uint32_t e) { return mrh::spill_base(t, entries) + e * mrh::SPILL_STRIDE; }
 extern "C" uint32_t slice(uint32_t b, uint32_t n) { return mrh::xcd_slice(b, n); }
@@ -29,7 +35,7 @@ def rules(tmp_path_factory):
     subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-Wall", "-Werror", "-I",
                     os.path.join(ROOT, "meturay_amd", "csrc"), str(d / "w.cpp"), "-o", so], check=True)
     lib = C.CDLL(so)
-    lib.blocks.argtypes = [C.c_uint64, C.c_uint32, C.c_uint32, C.c_uint64]
+    lib.blocks.argtypes = [C.c_uint64, C.c_int, C.c_uint32, C.c_uint64]
     lib.spill.argtypes, lib.spill.restype = [C.c_uint64, C.c_uint32, C.c_uint32], C.c_uint64
     return lib
 
@@ -40,7 +46,7 @@ def test_one_ray_kernels_fill_every_xcd(rules, block, most):
     """A one-ray-per-lane kernel's rays i, i + grid * block, ...: with fewer
     rays than threads the XCDs' shares differ by eight blocks at most."""
     for n in SIZES:
-        grid = rules.blocks(n, 64, block, most)
+        grid = rules.blocks(n, 0, block, most)
         assert grid % 8 == 0 and 8 <= grid <= (most + 7) // 8 * 8
         assert sorted(rules.slice(b, grid) for b in range(grid)) == list(range(grid))
         if n > grid * block:
@@ -52,6 +58,46 @@ def test_one_ray_kernels_fill_every_xcd(rules, block, most):
         assert sum(share) == n
         # up to 7 blocks that round the grid up are empty, one is half full
         assert max(share) - min(share) <= 8 * block, (n, share)
+
+
+def split(rules, n, grid, waves):
+    out = (C.c_uint32 * 2)()
+    rules.split(n, grid, waves, out)
+    return out[0], out[1]
+
+
+@pytest.mark.parametrize("block", [128, 256, 512])
+@pytest.mark.parametrize("most", [8, 256, MOST])
+@pytest.mark.parametrize("exact", [1, 0])
+def test_streaming_walk_takes_every_ray_once_on_all_xcds(rules, block, most, exact):
+    """Groups of a streaming walk, in a grid made for its rays (a cast) and in
+    one made for more of them (a later bounce of a frame)."""
+    waves = block // 64
+    for n in SIZES:
+        grid = rules.blocks(n if exact else 2_100_000, 1, block, most)
+        group, used = split(rules, n, grid, waves)
+        assert group in (16, 32, 64) and used % 8 == 0 and 8 <= used <= grid
+        assert sorted(rules.slice(b, used) for b in range(used)) == list(range(used))
+        stride = used * waves * group
+        if group < 64:
+            assert stride >= n   # the walk's first lots do not reach a second stride
+        share = [0] * 8          # a wave's rays: [g, g + group) for g = wave * group, + stride, ...
+        for b in range(used):
+            lo = rules.slice(b, used) * waves * group
+            share[b % 8] += max(0, min(n, lo + waves * group) - lo)
+        assert sum(share) == min(n, stride)
+        if n <= stride:
+            assert max(share) - min(share) <= 8 * waves * group, (n, share)
+
+
+def test_few_rays_spread_only_as_far_as_it_pays(rules):
+    """Waves of fewer than 64 rays are made for the chip's idle SIMDs, not
+    instead of full ones: 140,000 rays are 2,188 full waves, two a SIMD."""
+    for n, group in ((1, 16), (32_768, 16), (32_769, 32), (65_536, 32), (65_537, 64), (140_000, 64), (300_000, 64),
+                     (2_000_000, 64)):
+        grid = rules.blocks(n, 1, 256, MOST)
+        assert split(rules, n, grid, 4)[0] == group, n
+        assert split(rules, n, MOST, 4)[0] == group, n
 
 
 @pytest.mark.parametrize("width,lds,counting,streams", [(4, 8, 0, 1), (4, 24, 0, 1), (4, 0, 0, 0), (4, 8, 1, 0),

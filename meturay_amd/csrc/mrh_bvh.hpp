@@ -13,7 +13,7 @@
 #pragma once
 
 #include "mrh_internal.hpp"
-#include "mrh_walk.hpp"
+#include "mrh_shapes.hpp"
 
 #include <cfloat>
 

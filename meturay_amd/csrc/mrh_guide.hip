@@ -353,8 +353,7 @@ __device__ __forceinline__ float svo_filter_node(uint32_t node, float parent_mea
     return m;
 }
 
-// A wave takes a node of the levels up to `base` (two above the leaves) and
-// climbs to the first ancestor with samples in each of its empty bins (the
+// A wave takes a node of the levels up to `base` (svo_filter_base) and climbs to the first ancestor with samples in each of its empty bins (the
 // root: 0).  From a node of level `base` it goes on down to the node's
 // children and grandchildren with the means in registers, and writes their
 // final values; the means of higher nodes go to the radiance array first
@@ -1289,7 +1288,7 @@ int32_t svo_filter(mrh_context* ctx, mrh_svo* s)
                        s->lvl_off[l], c, (const uint32_t*)s->first_child, (const uint32_t*)s->child_mask, s->sum,
                        s->cnt));
     }
-    const uint32_t base = s->depth >= 2 ? s->depth - 2 : 0;
+    const uint32_t base = svo_filter_base(s->depth, s->lvl_count);
     const uint32_t base_off = s->lvl_off[base], base_end = s->lvl_off[base + 1];
     MRH_TRY(launch(ctx, "svo_filter", dim3(stride_grid(ctx, (uint64_t)base_end * GUIDE_BINS, 256)), dim3(256), 0,
                    k_svo_filter, base_off, base_end, (const uint32_t*)s->parent, (const uint32_t*)s->first_child,

@@ -1,6 +1,6 @@
-"""Launch shapes of the traversal kernels (mrh_walk.hpp) on the CPU: which
-block takes which rays is an integer rule, compiled here with the host
-compiler.  Every ray is taken once, and no XCD idles beside a full one."""
+"""Launch shapes (mrh_shapes.hpp) on the CPU: integer rules, compiled here with
+the host compiler.  Every ray is taken once, and no XCD idles beside a full
+one; the octree filter's waves go down only where there are many of them."""
 import ctypes as C
 import os
 import subprocess
@@ -13,7 +13,7 @@ SIZES = [1, 15, 16, 17, 63, 64, 65, 255, 256, 257, 1000, 5001, 20_000, 65_536, 1
 MOST = 256 * 8   # blocks of the whole chip at eight a CU
 
 SRC = r"""
-#include "mrh_walk.hpp"
+#include "mrh_shapes.hpp"
 extern "C" uint32_t blocks(uint64_t n, int stream, uint32_t block, uint64_t most) { return mrh::trace_blocks(n, stream != 0, block, most); }
 extern "C" void split(uint32_t n, uint32_t blocks, uint32_t waves, uint32_t* out)
 {
@@ -23,6 +23,7 @@ extern "C" void split(uint32_t n, uint32_t blocks, uint32_t waves, uint32_t* out
 }
 extern "C" int streams(uint32_t w, uint32_t lds, int counting) { return mrh::trace_streams(w, lds, counting != 0); }
 extern "C" uint64_t spill(uint64_t t, uint32_t entries, uint32_t e) { return mrh::spill_base(t, entries) + e * mrh::SPILL_STRIDE; }
+extern "C" uint32_t base(uint32_t depth, const uint32_t* count) { return mrh::svo_filter_base(depth, count); }
 extern "C" uint32_t slice(uint32_t b, uint32_t n) { return mrh::xcd_slice(b, n); }
 """
 
@@ -116,3 +117,16 @@ def test_spilled_entries_of_a_wave_share_lines(rules, entries):
     for row in at:
         for w in range(0, threads, 64):
             assert row[w:w + 64] == list(range(row[w], row[w] + 64))
+
+
+@pytest.mark.parametrize("counts,base", [
+    ([1, 8], 1), ([1, 8, 64], 2), ([1, 8, 64, 512, 4096, 32768], 4), ([1, 8, 64, 512, 4095, 32760], 5),
+    ([1, 8, 64, 512, 4096, 32768, 262144], 4), ([1] * 11, 10),
+    ([1, 8, 60, 300, 1200, 5000, 20_000, 80_000, 200_000, 400_000, 800_000], 8)])
+def test_octree_filter_goes_down_from_a_level_of_many_nodes(rules, counts, base):
+    """One wave per node of the base level: at least 4096 of them, or none
+    that takes more than its own node."""
+    depth = len(counts) - 1
+    got = rules.base(depth, (C.c_uint32 * len(counts))(*counts))
+    assert got == base
+    assert got == depth or (depth - got <= 2 and counts[got] >= 4096)

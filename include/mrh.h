@@ -723,7 +723,10 @@ int32_t mrh_render_guided(mrh_context* ctx, mrh_scene* scene, const mrh_camera_d
  * product sampler draws the guide direction and gives the product pdf at
  * the BxDF's direction, and the weight is f cos / (r p_product + (1 - r)
  * p_bxdf).  The product sampler's draws are hashed by the ray's place in the
- * bounce, so product renders are not reproducible path for path. */
+ * bounce, so product renders are not reproducible path for path.
+ * The context keeps up to 4 GiB of a render's memory for the next one; the
+ * rest goes back when the call ends, and all of it when another allocation of
+ * the context finds the device full. */
 typedef struct {
     uint32_t iterations;        /* frames, 1..64 (1 = plain path tracing) */
     uint32_t svo_depth;         /* "OctreeLevel", 1..10 */

@@ -26,6 +26,11 @@ int32_t dmalloc(mrh_context* ctx, void** p, size_t bytes)
     if (ctx->fail_alloc_after > 0 && --ctx->fail_alloc_after == 0)
         return fail(ctx, MRH_ERR_OOM, "hipMalloc(%zu) failed: injected by fail_alloc_after", bytes);
     hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && ctx->wfpg_users == 0) {
+        (void)hipGetLastError();
+        wfpg_release(ctx, 0);
+        e = hipMalloc(p, bytes);
+    }
     if (e != hipSuccess) {
         (void)hipGetLastError();
         *p = nullptr;
@@ -33,6 +38,31 @@ int32_t dmalloc(mrh_context* ctx, void** p, size_t bytes)
                     "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
     }
     return MRH_OK;
+}
+
+void wfpg_release(mrh_context* ctx, size_t keep)
+{
+    for (;;) {
+        size_t held = ctx->wfpg_svo ? svo_bytes(ctx->wfpg_svo) : 0, most = held;
+        int slot = -1;   // the largest; -1: the octree
+        for (int i = SLOT_WFPG_TRIS; i <= SLOT_WFPG_BINS; i++) {
+            held += ctx->slot_bytes[i];
+            if (ctx->slot_bytes[i] > most) {
+                most = ctx->slot_bytes[i];
+                slot = i;
+            }
+        }
+        if (held <= keep) return;
+        (void)hipStreamSynchronize(ctx->stream);
+        if (slot < 0) {
+            mrh_svo_destroy(ctx->wfpg_svo);
+            ctx->wfpg_svo = nullptr;
+        } else {
+            (void)hipFree(ctx->slot_ptr[slot]);
+            ctx->slot_ptr[slot] = nullptr;
+            ctx->slot_bytes[slot] = 0;
+        }
+    }
 }
 
 int32_t scratch(mrh_context* ctx, MrhSlot slot, size_t bytes, void** out)

@@ -1124,6 +1124,12 @@ SvoView svo_view(const mrh_svo* s)
     return v;
 }
 
+size_t svo_bytes(const mrh_svo* s)
+{
+    return (size_t)s->cap * 32 + (size_t)s->rad_cap * (GUIDE_BINS * 20 + 4) + s->work_a_bytes + s->work_b_bytes +
+           s->bin_work_bytes;
+}
+
 static int32_t svo_reserve(mrh_svo* s, uint32_t nodes, bool radiance)
 {
     mrh_context* ctx = s->ctx;

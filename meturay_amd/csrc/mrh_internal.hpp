@@ -34,8 +34,8 @@ enum MrhSlot : int {
     SLOT_VOXEL,
     SLOT_WFPG_TRIS,    // field-traced guided renders: triangles, voxel records,
     SLOT_WFPG_VOXELS,  // node payload, per-ray arrays, path vertices and the
-    SLOT_WFPG_NODES,   // bins of a bounce
-    SLOT_WFPG_RAYS,
+    SLOT_WFPG_NODES,   // bins of a bounce; given back past WFPG_KEEP_BYTES
+    SLOT_WFPG_RAYS,    // (wfpg_release)
     SLOT_WFPG_VERTS,
     SLOT_WFPG_BINS,
     SLOT_COUNT
@@ -78,6 +78,8 @@ struct mrh_context {
     struct mrh_svo* guide_svo = nullptr;
     // voxel octree reused by field-traced guided renders
     struct mrh_svo* wfpg_svo = nullptr;
+    // calls that use the SLOT_WFPG_ slots or that octree at the moment
+    uint32_t wfpg_users = 0;
     // this device's fixed partition workspace (mrh_partition_by_key_noalloc);
     // null when its address lookup failed (the reason in noalloc_err)
     void* noalloc_scratch = nullptr;
@@ -107,8 +109,27 @@ int32_t fail(mrh_context* ctx, int32_t code, const char* fmt, ...);
 // the next call that grows the same slot.
 int32_t scratch(mrh_context* ctx, MrhSlot slot, size_t bytes, void** out);
 
-// Device allocation with error reporting.
+// Device allocation with error reporting.  When the device is out of memory,
+// what idle field-traced renders keep is given back first.
 int32_t dmalloc(mrh_context* ctx, void** p, size_t bytes);
+
+// What field-traced guided renders keep between calls (the SLOT_WFPG_ slots and
+// the context's voxel octree): freed largest first until `keep` bytes are left.
+// A 1024 x 768 x 4 spp render of depth 10 needs about 1.6 GB, and its next call
+// is 10 ms shorter for finding it; 1080p at 16 spp and depth 12 needs 15 GB
+// (8.5 GB more in product mode), beside which those 10 ms are nothing.
+constexpr size_t WFPG_KEEP_BYTES = (size_t)4 << 30;
+void wfpg_release(mrh_context* ctx, size_t keep);
+// Marks a call that uses them
+struct WfpgUse {
+    mrh_context* ctx;
+    explicit WfpgUse(mrh_context* c) : ctx(c) { ctx->wfpg_users++; }
+    ~WfpgUse() { ctx->wfpg_users--; }
+    WfpgUse(const WfpgUse&) = delete;
+    WfpgUse& operator=(const WfpgUse&) = delete;
+};
+// Device bytes an octree holds
+size_t svo_bytes(const struct mrh_svo* s);
 
 // Begin/end event pair around a launch when profiling is enabled.
 hipEvent_t prof_begin(mrh_context* ctx);

@@ -899,7 +899,7 @@ __global__ void k_wf_tris(const float4* __restrict__ leaves, uint32_t n, float* 
 // and the octree on every call, and the fields again as the bins grew: a
 // 3-iteration 1024x768 x 4 spp render took 25.6 ms with that and takes 15.8 ms
 // with the context's blocks, one host read a bounce less and the voxel count
-// taken once.
+// taken once.  wfpg_release bounds what is kept between calls.
 int32_t wf_block(mrh_context* ctx, WfState& w, MrhSlot slot, size_t bytes, char** p)
 {
     void* q = nullptr;
@@ -941,6 +941,7 @@ __global__ void k_wf_pair(const uint32_t* __restrict__ count, const uint32_t* __
 int32_t wf_bounce(mrh_context* ctx, Frame& f, const PathBuf& in, const HitBuf& hb, const ShadeReq& q)
 {
     WfState& w = *f.wf;
+    const WfpgUse use(ctx);   // the bins' block
     uint32_t n = 0;
     MRH_HIP_CHECK(ctx, hipMemcpyAsync(&n, f.counts + f.bounce, 4, hipMemcpyDeviceToHost, ctx->stream));
     MRH_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
@@ -1565,6 +1566,7 @@ int32_t render_wfpg(mrh_context* ctx, mrh_scene* s, const mrh_camera_desc* cd, c
     MRH_TRY(fill_u32(ctx, (uint32_t*)d_image, 0u, img_count));
     GuideState g;
     WfState w;
+    const WfpgUse use(ctx);
     int32_t rc = guide_init(ctx, s, total, p->max_depth, &gp, nullptr, false, g);
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (rc == MRH_OK && hipEventCreate(&e0) != hipSuccess) rc = fail(ctx, MRH_ERR_HIP, "event create");
@@ -1603,6 +1605,7 @@ int32_t render_wfpg(mrh_context* ctx, mrh_scene* s, const mrh_camera_desc* cd, c
     if (e1) (void)hipEventDestroy(e1);
     wf_free(w);
     guide_free(g);
+    wfpg_release(ctx, rc == MRH_ERR_OOM ? 0 : WFPG_KEEP_BYTES);
     return rc;
 }
 
@@ -1910,6 +1913,7 @@ int32_t mrh_tracer_destroy(mrh_tracer* t)
     if (t->smem) (void)hipFree(t->smem);
     guide_free(t->g);
     wf_free(t->w);
+    wfpg_release(t->ctx, WFPG_KEEP_BYTES);   // the bins' block is the context's
     delete t;
     return MRH_OK;
 }

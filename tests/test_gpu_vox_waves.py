@@ -51,7 +51,7 @@ def test_neighbouring_walls_do_not_wait_for_each_other(ctx, n):
     assert many < 8 * one, (one, many)
 
 
-@pytest.mark.parametrize("depth,n", [(2, 40), (3, 2000), (4, 300), (5, 4000), (6, 500)])
+@pytest.mark.parametrize("depth,n", [(2, 40), (2, 16000), (3, 2000), (4, 300), (5, 4000), (6, 500)])
 def test_payload_normals_of_full_and_sparse_leaves(ctx, oracle, depth, n):
     rng = np.random.default_rng(10 * depth + n)
     tris = soup(rng, n)
@@ -60,6 +60,7 @@ def test_payload_normals_of_full_and_sparse_leaves(ctx, oracle, depth, n):
     tris = np.ascontiguousarray(tris[area > 1e-9])   # a degenerate triangle has no normal
     cube = cube_of(oracle, tris, depth)
     codes, prims = oracle.voxelize(tris, cube, depth, prims=True)
+    assert n < 16000 or len(codes) > 8 * 1536   # more than a block stages anything of
     svo, o = build_both(ctx, oracle, codes, cube, depth)
     verts = surface_vertices(rng, tris, 400)
     d_t, d_c, d_p, d_v = dev(tris.reshape(-1)), dev(codes), dev(prims), dev(verts.reshape(-1))

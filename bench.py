@@ -39,17 +39,17 @@ TRACE_SEG_BYTES, FRAME_SEG_BYTES, NODE_BYTES, TRI_BYTES = 44, 212, 32, 36
 PROFILES = os.path.join(ROOT, "profiles")
 
 
-def recorded_traffic(kernel: str, width: int, lds: int):
+def recorded_traffic(kernel: str, width: int, lds: int, bpc: int):
     """HBM bytes per launch of `kernel` measured by the rocprofv3 FETCH_SIZE /
-    WRITE_SIZE runs recorded in profiles/ for the same tree width and LDS
-    stack depth, or None."""
+    WRITE_SIZE runs recorded in profiles/ for the same tree width, LDS stack
+    depth and blocks per CU, or None."""
     import glob
     import re
-    pat = re.compile(r"^bench-traffic: (\S+) width=(\d+) lds=(\d+) bytes_per_launch=(\d+)", re.M)
+    pat = re.compile(r"^bench-traffic: (\S+) width=(\d+) lds=(\d+) bpc=(\d+) bytes_per_launch=(\d+)", re.M)
     for f in sorted(glob.glob(os.path.join(PROFILES, "*.md"))):
         for m in pat.finditer(open(f).read()):
-            if m.group(1) == kernel and (int(m.group(2)), int(m.group(3))) == (width, lds):
-                return int(m.group(4)), os.path.basename(f)
+            if m.group(1) == kernel and tuple(int(m.group(k)) for k in (2, 3, 4)) == (width, lds, bpc):
+                return int(m.group(5)), os.path.basename(f)
     return None
 
 
@@ -749,7 +749,7 @@ def main():
     frame_s = t_total / args.steps
     frame_with = (FRAME_SEG_BYTES * st.segments + tree_bytes) / frame_s / 1e9
     frame_without = FRAME_SEG_BYTES * st.segments / frame_s / 1e9
-    traffic = recorded_traffic("trace_pt", width, lds)
+    traffic = recorded_traffic("trace_pt", width, lds, bpc)
     img_np = img.cpu().numpy()
     log(f"per ray: {stc.node_visits / stc.segments:.1f} binary node visits, "
         f"{stc.tri_tests / stc.segments:.2f} triangle tests ({stw.node_visits / stw.segments:.1f} visits of "

@@ -654,7 +654,8 @@ constexpr uint32_t WALK_REFILL = 48;
 // lanes with work hold stack entries only, of which every step pops one.
 //
 // Bound by the node fetches (seven 16-byte loads of 64 lanes each keep the
-// CU's address unit 70 % busy) and by VALU issue (75 %).  Against the
+// CU's address unit 75 % busy; waves wait 36 % of their cycles) and by VALU
+// issue on partly filled waves (60 % busy).  Against the
 // one-ray-per-lane loop over traverse4: the frame above 16.5 -> 14.5 ms, the
 // casts 11.0 -> 6.6 ms.
 //

@@ -169,7 +169,7 @@ int32_t launch_trace_pt(mrh_context* ctx, uint64_t rays, const mrh_lbvh* b, cons
 // tree in local space (walk2l_stream; traverse_two_level for the other tree
 // widths and the counting variant); writes the instance too, and the
 // instance's HitKey override where it has one.  Five waves per SIMD: the walk
-// needs 89 registers.  1280x720 frame with NEE over 4096 instances: 8.48 ms
+// needs 90 registers.  1280x720 frame with NEE over 4096 instances: 8.48 ms
 // with one ray per lane, 6.65 ms with the stream (7.14 ms at six waves, which
 // spill).
 template <int W, int CAP, bool STATS, int L>
@@ -329,7 +329,7 @@ __global__ __launch_bounds__(256) void k_shade(PathBuf in, PathBuf out, HitBuf h
 
 // The same shade step with the partition done per block: a block takes a
 // tile of SHADE_TILE consecutive rays (coalesced key loads; 512, 1024 or
-// 2048, the "shade_tile" knob), counts them per HitKey batch in LDS, lays
+// 2048, the "shade_tile" knob, less for small frames), counts them per HitKey batch in LDS, lays
 // the tile's ray indices out batch by batch and shades them in that order,
 // so a wave nearly always runs one material while all ray-state lines of the
 // tile are fetched by the one block, once.  No global sort, no second pass
@@ -897,9 +897,9 @@ __global__ void k_wf_tris(const float4* __restrict__ leaves, uint32_t n, float* 
 // One block of the guide's memory: the context's grow-only slot, or memory of
 // the state's own.  Whole renders used to allocate and free their 30 buffers
 // and the octree on every call, and the fields again as the bins grew: a
-// 3-iteration 1024x768 x 4 spp render took 25.6 ms with that and takes 15.8 ms
-// with the context's blocks, one host read a bounce less and the voxel count
-// taken once.  wfpg_release bounds what is kept between calls.
+// 3-iteration 1024x768 x 4 spp render took 23.8 ms with that and 15.8 ms with
+// the context's blocks, one host read a bounce less and the voxel count taken
+// once.  wfpg_release bounds what is kept between calls.
 int32_t wf_block(mrh_context* ctx, WfState& w, MrhSlot slot, size_t bytes, char** p)
 {
     void* q = nullptr;

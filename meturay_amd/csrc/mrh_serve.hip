@@ -104,7 +104,7 @@ __global__ __launch_bounds__(256) void k_serve_raygen(const StepHdr* __restrict_
 
 // Closest hit of every queued ray in its own request's scene; camera rays
 // (depth 1) are clipped to the request's near/far planes.  Six waves per SIMD:
-// a lane's own tree takes the walk to 75 registers (12 guided and plain
+// a lane's own tree takes the walk to 80 registers (12 guided and plain
 // requests on two scenes: 9.26 / 9.28 / 8.87 ms at 8 / 7 / 6 waves, the first
 // two with spills; 10.2 ms with the one-ray-per-lane walk).
 template <int W, int CAP, int L>

@@ -14,7 +14,7 @@ namespace mrh {
 // 100,000 / 140,000 / 200,000 rays in 100 / 105 / 118 / 142 us; split up to four
 // waves a SIMD 111 / 116 / 118 / 142, up to eight 113 / 156 / 152 / 192.  500,000
 // triangles and 50,000 rays: 232 us; up to one wave a SIMD 248.
-constexpr uint32_t TRACE_MIN_GROUP = 16;
+constexpr uint32_t TRACE_MIN_SHIFT = 4, TRACE_MIN_GROUP = 1u << TRACE_MIN_SHIFT;
 constexpr uint32_t TRACE_SPLIT_WAVES = 2048;
 
 // Whether a traversal kernel runs the streaming walk, whose waves can take
@@ -51,12 +51,11 @@ struct WalkSplit {
 };
 constexpr WalkSplit walk_split(uint32_t n, uint32_t blocks, uint32_t waves)
 {
-    const uint64_t all = (uint64_t)blocks * waves, split = all < TRACE_SPLIT_WAVES ? all : TRACE_SPLIT_WAVES;
-    uint32_t group = 64;
-    while (group > TRACE_MIN_GROUP && trace_waves(n, group / 2) <= split) group /= 2;
-    const uint64_t need = (trace_waves(n, group) + waves - 1) / waves;
-    const uint64_t used = need ? (need + 7) & ~7ull : 8;
-    return {group, used < blocks ? (uint32_t)used : blocks};
+    const uint32_t all = blocks * waves, split = all < TRACE_SPLIT_WAVES ? all : TRACE_SPLIT_WAVES;
+    uint32_t shift = 6;   // of the group; shifts, since every wave of a launch starts here
+    while (shift > TRACE_MIN_SHIFT && (n - 1) >> (shift - 1) < split) shift--;
+    const uint32_t used = (n ? ((n - 1) >> shift) / waves + 8 : 8) & ~7u;
+    return {1u << shift, used < blocks ? used : blocks};
 }
 
 // Logical index of block `b` of `blocks` (a multiple of 8) that gives each of

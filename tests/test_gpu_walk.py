@@ -32,7 +32,8 @@ def _rays(m, seed):
 
 @pytest.mark.parametrize("lds", [8, 24])
 @pytest.mark.parametrize("n,m", [(1, 70), (2, 1), (700, 15), (700, 17), (5000, 65), (5000, 4097),
-                                 (60_000, 131_071), (60_000, 600_001)])
+                                 (5000, 32_769), (5000, 65_537),
+                                 (60_000, 131_071), (60_000, 300_001), (60_000, 600_001)])
 def test_stream_walk_equals_oracle(ctx, oracle, n, m, lds):
     tris, rays = _scene(n), _rays(m, n + m)
     old = ctx.tune_get("trace_lds_entries"), ctx.tune_get("trace_blocks_per_cu")
